@@ -240,29 +240,44 @@ struct Variant {
   surface_fn surface;
   ens_fn ens_plain, ens_phys;                    /* persistent ensemble stage kernels (null: no ensemble) */
   ens_surface_fn ens_surface;
+  bool sb;                                       /* compiled for one blending weight of the hybrid schemes */
   const char *name;
 };
 
-template <bool TKE, int NM, int SH, int SE, int SQV, int SQL, bool ENS = false, bool TERR = false>
+/* SB: compiled for equal blending weights b of the hybrid schemes.  A face's six stencil weights
+ * depend on the wind's sign and b only, so they are then formed once per face for all fields, not
+ * once per field group (20 of 390 vector instructions per level and wave of the plain stage); the
+ * results are the same bits. */
+template <bool TKE, int NM, int SH, int SE, int SQV, int SQL, bool ENS, bool TERR, bool SB>
 Variant make_variant(const char *name) {
   Variant v;
-  v.plain = stage_plain_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, false, TERR>, false>;
-  v.plain_emit = stage_plain_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, false, TERR>, true>;
-  v.phys = stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR>, false>;
-  v.phys_emit = stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR>, true>;
-  if constexpr (NM > 1) v.phys_nomp = stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR>, false, false>;
+  v.sb = SB;
+  v.plain = stage_plain_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, false, TERR, SB>, false>;
+  v.plain_emit = stage_plain_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, false, TERR, SB>, true>;
+  v.phys = stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR, SB>, false>;
+  v.phys_emit = stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR, SB>, true>;
+  if constexpr (NM > 1) v.phys_nomp = stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR, SB>, false, false>;
   else v.phys_nomp = v.phys;
-  v.surface = surface_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR>>;
+  v.surface = surface_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, TERR, SB>>;
   v.ens_plain = nullptr;
   v.ens_phys = nullptr;
   v.ens_surface = nullptr;
   if constexpr (ENS) {
-    v.ens_plain = ens_stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, false>, false>;
-    v.ens_phys = ens_stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true>, true>;
-    v.ens_surface = ens_surface_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true>>;
+    v.ens_plain = ens_stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, false, false, SB>, false>;
+    v.ens_phys = ens_stage_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, false, SB>, true>;
+    v.ens_surface = ens_surface_kernel<Cfg<TKE, NM, SH, SE, SQV, SQL, true, false, SB>>;
   }
   v.name = name;
   return v;
+}
+
+template <bool TKE, int NM, int SH, int SE, int SQV, int SQL, bool ENS = false, bool TERR = false>
+Variant pick_variant(const char *name) {
+  constexpr bool hyb = SH == 2 || SH == 3;                 /* schemes with a blending weight */
+  const bool sb = (!TKE || b_hyb == TKEAdvSelector_b_hyb) && (NM == 0 || b_hyb == moistureAdvSelectorQv_b);
+  if constexpr (hyb && (TKE || NM > 0))
+    if (sb) return make_variant<TKE, NM, SH, SE, SQV, SQL, ENS, TERR, true>(name);
+  return make_variant<TKE, NM, SH, SE, SQV, SQL, ENS, TERR, false>(name);
 }
 
 Variant g_var;
@@ -280,11 +295,11 @@ int select_variant(void) {
      * advection with the prognostic-TKE closure (dry, and the shallow-cumulus q_v/q_l set with
      * WENO5 liquid) and with the Smagorinsky closure (dry) */
     if (tke && nm == 0 && sh == 3 && se == 3) {
-      g_var = make_variant<true, 0, 3, 3, 3, 5, false, true>("dry+tke hyb56/hyb56 terrain-following");
+      g_var = pick_variant<true, 0, 3, 3, 3, 5, false, true>("dry+tke hyb56/hyb56 terrain-following");
     } else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 5) {
-      g_var = make_variant<true, 2, 3, 3, 3, 5, false, true>("moist2+tke hyb56/hyb56/hyb56/weno5 terrain-following");
+      g_var = pick_variant<true, 2, 3, 3, 3, 5, false, true>("moist2+tke hyb56/hyb56/hyb56/weno5 terrain-following");
     } else if (!tke && turbulenceSelector > 0 && nm == 0 && sh == 3) {
-      g_var = make_variant<false, 0, 3, 3, 3, 5, false, true>("dry smagorinsky hyb56 terrain-following");
+      g_var = pick_variant<false, 0, 3, 3, 3, 5, false, true>("dry smagorinsky hyb56 terrain-following");
     } else {
       fprintf(stderr, "select_variant: terrain-following grids run HYB56 advection with the prognostic-TKE closure "
                       "(dry, or q_v/q_l with WENO5 liquid) or the dry Smagorinsky closure\n");
@@ -293,21 +308,21 @@ int select_variant(void) {
     g_var_ok = 1;
     return FE_OK;
   }
-  if (tke && nm == 0 && sh == 3 && se == 3) { g_var = make_variant<true, 0, 3, 3, 3, 5, true>("dry+tke hyb56/hyb56"); g_var_ok = 1; }
-  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 5) { g_var = make_variant<true, 2, 3, 3, 3, 5, true>("moist2+tke hyb56/hyb56/hyb56/weno5"); g_var_ok = 1; }
-  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 2 && sql == 5) { g_var = make_variant<true, 2, 3, 3, 2, 5>("moist2+tke hyb56/hyb56/hyb34/weno5"); g_var_ok = 1; }
-  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 0) { g_var = make_variant<true, 2, 3, 3, 3, 0>("moist2+tke hyb56/.../upstream"); g_var_ok = 1; }
-  else if (tke && nm == 1 && sh == 3 && se == 3 && sqv == 3) { g_var = make_variant<true, 1, 3, 3, 3, 5>("moist1+tke hyb56"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 5 && se == 5) { g_var = make_variant<true, 0, 5, 5, 3, 5>("dry+tke weno5/weno5"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 2 && se == 2) { g_var = make_variant<true, 0, 2, 2, 3, 5>("dry+tke hyb34/hyb34"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 1 && se == 1) { g_var = make_variant<true, 0, 1, 1, 3, 5>("dry+tke quick/quick"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 0 && se == 0) { g_var = make_variant<true, 0, 0, 0, 3, 5>("dry+tke upstream"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 6 && se == 6) { g_var = make_variant<true, 0, 6, 6, 3, 5>("dry+tke centred2"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 4 && se == 4) { g_var = make_variant<true, 0, 4, 4, 3, 5>("dry+tke weno3"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 3 && se == 0) { g_var = make_variant<true, 0, 3, 0, 3, 5>("dry+tke hyb56/upstream"); g_var_ok = 1; }
-  else if (!tke && turbulenceSelector == 0 && nm == 0 && sh == 3) { g_var = make_variant<false, 0, 3, 3, 3, 5>("dry inviscid hyb56"); g_var_ok = 1; }
-  else if (!tke && turbulenceSelector > 0 && nm == 0 && sh == 3) { g_var = make_variant<false, 0, 3, 3, 3, 5, true>("dry smagorinsky hyb56"); g_var_ok = 1; }
-  else if (!tke && turbulenceSelector > 0 && nm == 2 && sh == 3 && sqv == 3 && sql == 5) { g_var = make_variant<false, 2, 3, 3, 3, 5>("moist2 smagorinsky hyb56/hyb56/weno5"); g_var_ok = 1; }
+  if (tke && nm == 0 && sh == 3 && se == 3) { g_var = pick_variant<true, 0, 3, 3, 3, 5, true>("dry+tke hyb56/hyb56"); g_var_ok = 1; }
+  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 5) { g_var = pick_variant<true, 2, 3, 3, 3, 5, true>("moist2+tke hyb56/hyb56/hyb56/weno5"); g_var_ok = 1; }
+  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 2 && sql == 5) { g_var = pick_variant<true, 2, 3, 3, 2, 5>("moist2+tke hyb56/hyb56/hyb34/weno5"); g_var_ok = 1; }
+  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 0) { g_var = pick_variant<true, 2, 3, 3, 3, 0>("moist2+tke hyb56/.../upstream"); g_var_ok = 1; }
+  else if (tke && nm == 1 && sh == 3 && se == 3 && sqv == 3) { g_var = pick_variant<true, 1, 3, 3, 3, 5>("moist1+tke hyb56"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 5 && se == 5) { g_var = pick_variant<true, 0, 5, 5, 3, 5>("dry+tke weno5/weno5"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 2 && se == 2) { g_var = pick_variant<true, 0, 2, 2, 3, 5>("dry+tke hyb34/hyb34"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 1 && se == 1) { g_var = pick_variant<true, 0, 1, 1, 3, 5>("dry+tke quick/quick"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 0 && se == 0) { g_var = pick_variant<true, 0, 0, 0, 3, 5>("dry+tke upstream"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 6 && se == 6) { g_var = pick_variant<true, 0, 6, 6, 3, 5>("dry+tke centred2"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 4 && se == 4) { g_var = pick_variant<true, 0, 4, 4, 3, 5>("dry+tke weno3"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 3 && se == 0) { g_var = pick_variant<true, 0, 3, 0, 3, 5>("dry+tke hyb56/upstream"); g_var_ok = 1; }
+  else if (!tke && turbulenceSelector == 0 && nm == 0 && sh == 3) { g_var = pick_variant<false, 0, 3, 3, 3, 5>("dry inviscid hyb56"); g_var_ok = 1; }
+  else if (!tke && turbulenceSelector > 0 && nm == 0 && sh == 3) { g_var = pick_variant<false, 0, 3, 3, 3, 5, true>("dry smagorinsky hyb56"); g_var_ok = 1; }
+  else if (!tke && turbulenceSelector > 0 && nm == 2 && sh == 3 && sqv == 3 && sql == 5) { g_var = pick_variant<false, 2, 3, 3, 3, 5>("moist2 smagorinsky hyb56/hyb56/weno5"); g_var_ok = 1; }
   return g_var_ok ? FE_OK : FE_ERR_UNSUPPORTED;
 }
 

@@ -302,6 +302,7 @@ int fe_ens_add_member(void) {
         fprintf(stderr, "fe_ens_add_member: members must share the physics-stage schedule (physics_oneRKonly)\n");
         return -FE_ERR_UNSUPPORTED;
       }
+    if (E.var.sb && !g_var.sb) E.var = g_var;    /* a member whose blending weights differ: kernels for any weights */
   } else {
     E.var = g_var;
     E.have_var = true;

@@ -49,6 +49,7 @@ constexpr int RW = TX + 2 * HH, RH = TY + 2 * HH;      /* raw plane with 3-cell 
 constexpr int DW = TX + 2, DH = TY + 2;                /* ring-1 region [-1,TX] x [-1,TY]     */
 constexpr int NHALO = RW * RH - TX * TY;               /* halo cells of the raw plane (<= NT) */
 constexpr int NR1 = DW * DH - TX * TY;                 /* ring-1 cells, listed first          */
+constexpr int NFP = 8;                                 /* fields per row of the ring column's fluxes (16-byte rows) */
 /* third word of a raw (stride 0) buffer resource on CDNA: 32-bit data format, no swizzle */
 constexpr int FE_RSRC_W3 = 0x00020000;
 static_assert(NHALO <= NT, "one halo cell per thread");
@@ -251,8 +252,9 @@ __device__ __forceinline__ float pprime(const StepArgs &a, float rth, float mf, 
 }
 
 
-template <bool TKE_, int NM_, int SH_, int SE_, int SQV_, int SQL_, bool PHYS_, bool TERR_ = false>
+template <bool TKE_, int NM_, int SH_, int SE_, int SQV_, int SQL_, bool PHYS_, bool TERR_ = false, bool SB_ = false>
 struct Cfg {
+  static constexpr bool SB = SB_;             /* one blending weight b of the hybrid schemes for every field */
   static constexpr bool TKE = TKE_;
   static constexpr bool TERR = TERR_;         /* terrain-following grid: per-column metrics and base state */
   static constexpr int NM = NM_;
@@ -273,19 +275,38 @@ struct Cfg {
 /* LDS-qualified float: stencil reads through it compile to ds_read (paired where the offsets
  * allow) rather than flat loads whose address space the compiler would have to prove */
 typedef __attribute__((address_space(3))) float SRD;
+/* LDS address p + K floats, added where the compiler cannot see it: reads at small constant
+ * offsets from the result share it as their base.  Left alone, the compiler folds every constant
+ * into each read and then adds a base of its own per paired read (whose offsets reach 255 floats):
+ * 40 adds per level and wave of the plain stage. */
+template <int K>
+__device__ __forceinline__ const SRD *lds_at(const SRD *p) {
+  unsigned r;
+  asm("v_add_u32 %0, %2, %1" : "=v"(r) : "v"((unsigned)(unsigned long)p), "n"(K * 4));
+  return (const SRD *)(unsigned long)r;
+}
+/* v of the next lane in x (a wave holds whole tile rows); the last lane of a row gets edge */
+__device__ __forceinline__ float lane_up(float v, float edge, int tx) {
+  constexpr int WAVE_SHL1 = 0x130;         /* DPP: lane i takes lane i + 1; the last lane keeps 'old' */
+  const int r = __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge), __builtin_bit_cast(int, v), WAVE_SHL1, 0xf, 0xf, false);
+  if constexpr (TX == 64) return __builtin_bit_cast(float, r);
+  else return tx == TX - 1 ? edge : __builtin_bit_cast(float, r);
+}
 template <class C, int F, int FE = C::NF>
 struct FaceLoop {
-  __device__ __forceinline__ static void xf(float (*raw)[RH][RW], float (*gx)[TY][TX + 1], int fy, int fx, float U, const float *omb) {
+  /* x face fx = TX of row fy (the tile's ring column) */
+  __device__ __forceinline__ static void xr(float (*raw)[RH][RW], float *g, int fy, float U, const float *omb) {
     if constexpr (F < FE) {
-      const SRD *r = (const SRD *)&raw[F][fy + HH][fx];
-      gx[F][fy][fx] = face_flux<C::template sch<F>(), C::PHYS>(U, omb[F], r[0], r[1], r[2], r[3], r[4], r[5]);
-      FaceLoop<C, F + 1, FE>::xf(raw, gx, fy, fx, U, omb);
+      const SRD *r = lds_at<F * RH * RW>((const SRD *)&raw[0][fy + HH][TX]);
+      g[F] = face_flux<C::template sch<F>(), C::PHYS>(U, omb[F], r[0], r[1], r[2], r[3], r[4], r[5]);
+      FaceLoop<C, F + 1, FE>::xr(raw, g, fy, U, omb);
     }
   }
   __device__ __forceinline__ static void yf(float (*raw)[RH][RW], float (*gy)[TY + 1][TX], int fy, int fx, float V, const float *omb) {
     if constexpr (F < FE) {
-      const SRD *r = (const SRD *)&raw[F][fy][fx + HH];
-      gy[F][fy][fx] = face_flux<C::template sch<F>(), C::PHYS>(V, omb[F], r[0], r[RW], r[2 * RW], r[3 * RW], r[4 * RW], r[5 * RW]);
+      const SRD *o = (const SRD *)&raw[0][fy][fx + HH], *r = lds_at<F * RH * RW>(o);
+      gy[F][fy][fx] = face_flux<C::template sch<F>(), C::PHYS>(V, omb[F], r[0], r[RW], r[2 * RW], r[3 * RW],
+                                                               o[F * RH * RW + 4 * RW], o[F * RH * RW + 5 * RW]);
       FaceLoop<C, F + 1, FE>::yf(raw, gy, fy, fx, V, omb);
     }
   }
@@ -298,6 +319,61 @@ struct FaceLoop {
   }
 };
 
+/* The own cell's x and y neighbours in the planes, i-3, i-2, i-1, i+1, i+2 of fields [F0, F1)
+ * (the cell itself, c, is in its register window), and the fluxes through its low faces. */
+template <class C, int F0, int F1>
+struct OwnStencil {
+  float x[F1 - F0][5], y[F1 - F0][5];
+  template <int F = F0>
+  __device__ __forceinline__ void load(const SRD *o) {    /* o = &raw[0][ty][tx] */
+    if constexpr (F < F1) {
+      const SRD *r = lds_at<F * RH * RW>(o);
+#pragma unroll
+      for (int j = 0; j < 5; ++j) {
+        const int d = j < 3 ? j : j + 1;
+        x[F - F0][j] = r[HH * RW + d];
+        y[F - F0][j] = d < 5 ? r[d * RW + HH] : o[F * RH * RW + d * RW + HH];
+      }
+      load<F + 1>(o);
+    }
+  }
+  template <int F = F0>
+  __device__ __forceinline__ void flux(const float *c, float U, float V, const float *omb, float *fx, float *fy) const {
+    if constexpr (F < F1) {
+      constexpr int SC = C::template sch<F>(), N = F - F0;
+      fx[F] = face_flux<SC, C::PHYS>(U, omb[F], x[N][0], x[N][1], x[N][2], c[F], x[N][3], x[N][4]);
+      fy[F] = face_flux<SC, C::PHYS>(V, omb[F], y[N][0], y[N][1], y[N][2], c[F], y[N][3], y[N][4]);
+      flux<F + 1>(c, U, V, omb, fx, fy);
+    }
+  }
+};
+/* Advective fluxes of every field through the own cell's low x and y faces; dr: the rho^-1 plane
+ * (terrain: D rho^-1) around the cell, rc its value at the cell, hxD, hyD: 0.5 D/dx, 0.5 D/dy (0.5/dx, 0.5/dy).
+ * The stages issue about one vector instruction in two cycles of their two waves per SIMD, and
+ * every other instruction takes an issue slot of the wave too, so what counts here is their number:
+ * the cell's own values come from registers, five neighbours per field and direction from LDS at
+ * one base per field, the x flux of the next cell from the neighbouring lane (lane_up), and only
+ * the y fluxes go through LDS.  512 x 512 x 128 dry: 391 -> 336 vector and 81 -> 71 LDS
+ * instructions per level and wave of the plain stage, 0.643 -> 0.606 ms (3.7 TB/s of its HBM
+ * traffic); physics stage 1.099 -> 1.061 ms; over a hill (256 x 256 x 128) 0.249 -> 0.215 ms. */
+template <class C>
+__device__ __forceinline__ void own_faces(float (*raw)[RH][RW], const float (*dr)[DW], int ty, int tx, const float *c,
+                                          float rc, float hxD, float hyD, const float *omb, float *fx, float *fy) {
+  const SRD *o = (const SRD *)&raw[0][ty][tx];
+  constexpr int FH = C::NM > 0 ? 4 : C::NF;    /* moist: in two halves, which keeps the second's neighbours out of registers */
+  OwnStencil<C, 0, FH> n;
+  n.load(o);
+  const float U = hxD * (n.x[1][2] * dr[ty + 1][tx] + c[1] * rc);
+  const float V = hyD * (n.y[2][2] * dr[ty][tx + 1] + c[2] * rc);
+  n.flux(c, U, V, omb, fx, fy);
+  if constexpr (FH < C::NF) {
+    __builtin_amdgcn_sched_barrier(0);
+    OwnStencil<C, FH, C::NF> m;
+    m.load(o);
+    m.flux(c, U, V, omb, fx, fy);
+  }
+}
+
 /* Advective fluxes of fields [F0, F1) through the tile's ring faces: face i of the y face
  * row y = TY and face i of the x face column x = TX. */
 template <class C, int F0, int F1>
@@ -308,11 +384,11 @@ __device__ __forceinline__ void ring_faces_y(float (*raw)[RH][RW], float (*gy)[T
   FaceLoop<C, F0, F1>::yf(raw, gy, fy, fx, V, omb);
 }
 template <class C, int F0, int F1>
-__device__ __forceinline__ void ring_faces_x(float (*raw)[RH][RW], float (*gx)[TY][TX + 1], const float (*dr)[DW], int i,
+__device__ __forceinline__ void ring_faces_x(float (*raw)[RH][RW], float (*gxr)[NFP], const float (*dr)[DW], int i,
                                              float hxD, const float *omb) {
   const int fx = TX, fy = i;
   const float U = hxD * (raw[1][fy + HH][fx + HH - 1] * dr[fy + 1][fx] + raw[1][fy + HH][fx + HH] * dr[fy + 1][fx + 1]);
-  FaceLoop<C, F0, F1>::xf(raw, gx, fy, fx, U, omb);
+  FaceLoop<C, F0, F1>::xr(raw, gxr[fy], fy, U, omb);
 }
 
 /* SGS stress pieces on a face-located cell (cuda_sgsTurbDevice.cu:60-367).  All
@@ -694,7 +770,7 @@ struct Tile {
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       int s = (f < 5) ? C::SH : ((C::TKE && f == C::IE) ? C::SE : (f == C::IQV ? C::SQV : C::SQL));
-      float bb = (f < 5) ? a.bh : ((C::TKE && f == C::IE) ? a.be : a.bqv);
+      float bb = (C::SB || f < 5) ? a.bh : ((C::TKE && f == C::IE) ? a.be : a.bqv);
       omb[f] = (s == 3 || s == 2) ? bb : 0.f;
     }
   }
@@ -769,7 +845,7 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
   __shared__ float raw[NF][RH][RW];
   __shared__ float dvr[DH][DW];          /* rho^-1 of the ring-1 region (terrain-following grids: D rho^-1) */
   __shared__ float dvp[DH][DW];
-  __shared__ float gx[NF][TY][TX + 1];
+  __shared__ __align__(16) float gxr[TY][NFP];      /* x fluxes of the ring column x = TX */
   __shared__ float gy[NF][TY + 1][TX];
   /* velocities u,v,w rotate over four levels, theta and moisture over three */
   __shared__ float velm[PH ? 4 : 1][PH ? 3 : 1][DH][DW];
@@ -1106,6 +1182,7 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
     /* horizontal p' differences of the own cell, read here so that the p' plane
      * is free to be rewritten in the next level's first phase */
     float t11 = 0.f, t21 = 0.f, t22 = 0.f;          /* own-cell SGS stresses, P2 -> P3 */
+    float fx[NF], fy[NF];                           /* fluxes through the own cell's low faces, P2 -> P3 */
     const float pgx = 0.5f * a.dXi * (dvp[ty + 1][tx + 2] - dvp[ty + 1][tx]);
     const float pgy = 0.5f * a.dYi * (dvp[ty + 2][tx + 1] - dvp[ty][tx + 1]);
     {
@@ -1117,20 +1194,22 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
       const float (*dfv)[DW] = dvr;
       /* own x face (low face of the own cell) and own y face */
       {
-        float U = hxD * (raw[1][ty + HH][tx + HH - 1] * dfv[ty + 1][tx] + raw[1][ty + HH][tx + HH] * dfv[ty + 1][tx + 1]);
-        FaceLoop<C, 0>::xf(raw, gx, ty, tx, U, omb);
-        float V = hyD * (raw[2][ty + HH - 1][tx + HH] * dfv[ty][tx + 1] + raw[2][ty + HH][tx + HH] * dfv[ty + 1][tx + 1]);
-        FaceLoop<C, 0>::yf(raw, gy, ty, tx, V, omb);
+        float c[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = win[f][3];
+        own_faces<C>(raw, dfv, ty, tx, c, C::TERR ? dfv[ty + 1][tx + 1] : rin, hxD, hyD, omb, fx, fy);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) gy[f][ty][tx] = fy[f];
       }
       /* ring faces (on the 64 x 8 tile half of the fields per job row) */
       {
         constexpr int HF = PL.split ? NF / 2 : NF;
         int i;
         if (on_job(PL.rfy[0], wave, lane, i)) ring_faces_y<C, 0, HF>(raw, gy, dfv, i, hyD, omb);
-        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, HF>(raw, gx, dfv, i, hxD, omb);
+        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, HF>(raw, gxr, dfv, i, hxD, omb);
         if constexpr (PL.split) {
           if (on_job(PL.rfy[1], wave, lane, i)) ring_faces_y<C, HF, NF>(raw, gy, dfv, i, hyD, omb);
-          if (on_job(PL.rfx[1], wave, lane, i)) ring_faces_x<C, HF, NF>(raw, gx, dfv, i, hxD, omb);
+          if (on_job(PL.rfx[1], wave, lane, i)) ring_faces_x<C, HF, NF>(raw, gxr, dfv, i, hxD, omb);
         }
       }
       if constexpr (PH) {
@@ -1238,7 +1317,8 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
       const float rinp = frcp(win[0][4]);
       float dxy[NF], gzhi[NF], F[NF];
 #pragma unroll
-      for (int f = 0; f < NF; ++f) dxy[f] = (gx[f][ty][tx + 1] - gx[f][ty][tx]) + (gy[f][ty + 1][tx] - gy[f][ty][tx]);
+      for (int f = 0; f < NF; ++f)
+        dxy[f] = (lane_up(fx[f], ((const SRD *)gxr[ty])[f], tx) - fx[f]) + (((const SRD *)&gy[f][ty][tx])[TX] - fy[f]);
       dyn_tendency<C, 7>(a, z, C::TERR ? trow : dyn_rows<C>(a, z, (unsigned)col), win, rin, rinp, pz[0], pz[2], pgx, pgy, dxy,
                          gzlo, gzhi, omb, F);
       const float rho = win[0][3];
@@ -1454,8 +1534,14 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
   __shared__ float raw[2][NF][RH][RW];
   __shared__ float dvr[2][DH][DW];       /* rho^-1 of the ring-1 region (terrain-following grids: D rho^-1) */
   __shared__ float dvp[2][DH][DW];
-  __shared__ float gx[2][NF][TY][TX + 1];
+  __shared__ __align__(16) float gxr[2][TY][NFP];   /* x fluxes of the ring column x = TX */
   __shared__ float gy[2][NF][TY + 1][TX];
+  /* x fluxes through the own cells' low faces: carried in registers from P2 to the next
+   * iteration's P3, or through LDS when moist (two more fields, and no registers left) */
+  constexpr bool FXR = C::NM == 0;
+  /* RK base of P3's level loaded one iteration ahead, or (moist, for registers) at the start of its own */
+  constexpr bool BSA = C::NM == 0;
+  __shared__ float gxo[FXR ? 1 : 2][FXR ? 1 : NF][FXR ? 1 : TY][FXR ? 1 : TX];
 
   constexpr RingPlan PL = PLAN_PLAIN;
   const Tile<C> T(a, tp, PL.r1);
@@ -1471,7 +1557,8 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
    *   hv[l+S]: halo cell, level it+l;  bs[S]: RK base of level it-2 (bs[S+1] in flight);
    *   pp[S..S+3]: own p' of levels it-3..it;  ri[S..S+2]: own rho^-1 of levels it-2..it;
    *   pg[S]: horizontal p' differences of level it-2 (pg[S+1] written for it-1);
-   *   gz[S]: z flux through the lower face of level it-2 (gz[S+1] its upper face). */
+   *   gz: z flux through the lower face of level it-2;
+   *   fx[S]: x flux through the own cell's low face at level it-2 (fx[S+1] written for it-1). */
   /* A z segment [zs, ze) other than the first starts its pipeline at it0 = zs - 2: P1
    * of levels zs-2 and zs-1 and P2/P3 of level zs-1 run without output, so that p',
    * the plane buffers and the z flux through the segment's lower face are in place
@@ -1507,11 +1594,15 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
   };
   if (it0 == 0) init(0);
   else init(it0);
-  float bs[3][NF], gz[3][NF];
+  float bs[BSA ? 3 : 1][NF], gz[NF], fx[FXR ? 3 : 1][FXR ? NF : 1];
 #pragma unroll
-  for (int l = 0; l < 3; ++l)
+  for (int f = 0; f < NF; ++f) {
+    gz[f] = 0.f;
+    for (int l = 0; l < (BSA ? 3 : 1); ++l) bs[l][f] = 0.f;
+  }
+  if constexpr (FXR)
 #pragma unroll
-    for (int f = 0; f < NF; ++f) bs[l][f] = gz[l][f] = 0.f;
+    for (int f = 0; f < NF; ++f) fx[0][f] = fx[1][f] = fx[2][f] = 0.f;
   float pp[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
   float ri[4] = {0.f, 0.f, 0.f, 0.f};
   /* terrain-following grids: P1's base-state rows and D of level it (own column and ring-1
@@ -1559,10 +1650,15 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
       }
     }
     /* ---- loads for the next level: RK base of level it-1, own level it+2, halo level it+2 ---- */
-    if (z2 >= 0 && z2 < Nz && !a.emitF && !T.baseIn) {
-      const unsigned o2 = (unsigned)z2 * pb + colb;
+    if constexpr (BSA) {
+      if (z2 >= 0 && z2 < Nz && !a.emitF && !T.baseIn) {
+        const unsigned o2 = (unsigned)z2 * pb + colb;
 #pragma unroll
-      for (int f = 0; f < NF; ++f) bs[S + 1][f] = T.ld_bs(f, o2);
+        for (int f = 0; f < NF; ++f) bs[S + 1][f] = T.ld_bs(f, o2);
+      }
+    } else if (z3 >= zs && !a.emitF && !T.baseIn) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) bs[0][f] = T.ld_bs(f, o3);
     }
     {
       float t[NF];
@@ -1608,56 +1704,67 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
       const float Dz = C::TERR ? 1.f : prof(a, PR_D, z2);
       const float hxD = 0.5f * a.dXi * Dz, hyD = 0.5f * a.dYi * Dz;
       {
-        float U = hxD * (rw[1][ty + HH][tx + HH - 1] * dr[ty + 1][tx] + rw[1][ty + HH][tx + HH] * dr[ty + 1][tx + 1]);
-        FaceLoop<C, 0>::xf(rw, gx[b2], ty, tx, U, T.omb);
-        float V = hyD * (rw[2][ty + HH - 1][tx + HH] * dr[ty][tx + 1] + rw[2][ty + HH][tx + HH] * dr[ty + 1][tx + 1]);
-        FaceLoop<C, 0>::yf(rw, gy[b2], ty, tx, V, T.omb);
+        float c[NF], fxn[NF], fy[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) c[f] = win[f][4 + S];
+        own_faces<C>(rw, dr, ty, tx, c, C::TERR ? dr[ty + 1][tx + 1] : ri[S + 1], hxD, hyD, T.omb, fxn, fy);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          gy[b2][f][ty][tx] = fy[f];
+          if constexpr (FXR) fx[S + 1][f] = fxn[f];
+          else gxo[b2][f][ty][tx] = fxn[f];
+        }
       }
       /* ring faces, all fields per job row (splitting them over more waves costs more issue
        * slots than it saves in barrier wait) */
       {
         int i;
         if (on_job(PL.rfy[0], wave, lane, i)) ring_faces_y<C, 0, NF>(rw, gy[b2], dr, i, hyD, T.omb);
-        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, NF>(rw, gx[b2], dr, i, hxD, T.omb);
+        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, NF>(rw, gxr[b2], dr, i, hxD, T.omb);
       }
     }
 
     /* ---- P3: own cell of level it-2 ---- */
     if (z3 >= zlo) {
-      float dxy[NF], F[NF];
+      float dxy[NF], gzhi[NF], F[NF];
       float (*wv)[9] = win;
       float w7[NF][7];
 #pragma unroll
       for (int f = 0; f < NF; ++f)
 #pragma unroll
         for (int j = 0; j < 7; ++j) w7[f][j] = wv[f][j + S];
+      float xr[NFP];
+#pragma unroll
+      for (int f = 0; f < NFP; ++f) xr[f] = f < NF ? ((const SRD *)gxr[b1][ty])[f] : 0.f;
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        const SRD *px = (const SRD *)&gx[b1][f][ty][tx], *py = (const SRD *)&gy[b1][f][ty][tx];
-        dxy[f] = (px[1] - px[0]) + (py[TX] - py[0]);
+        const SRD *py = (const SRD *)&gy[b1][f][ty][tx];
+        float px;
+        if constexpr (FXR) px = fx[S][f];
+        else px = ((const SRD *)&gxo[b1][f][ty][tx])[0];
+        dxy[f] = (lane_up(px, xr[f], tx) - px) + (py[TX] - py[0]);
       }
-      dyn_tendency<C, 7>(a, z3, C::TERR ? trow : dyn_rows<C>(a, z3, (unsigned)T.col), w7, ri[S], ri[S + 1], pp[S], pp[S + 2], pg[S][0],
-                         pg[S][1], dxy, gz[S], gz[S + 1],
-                         T.omb, F);
+      dyn_tendency<C, 7>(a, z3, C::TERR ? trow : dyn_rows<C>(a, z3, (unsigned)T.col), w7, ri[S], ri[S + 1], pp[S], pp[S + 2], pg[S][0], pg[S][1],
+                         dxy, gz, gzhi, T.omb, F);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) gz[f] = gzhi[f];
       if (z3 >= zs) {                                 /* uniform: not a warm-up level */
         if (T.active) {
           float b0[NF];
 #pragma unroll
-          for (int f = 0; f < NF; ++f) b0[f] = T.baseIn ? win[f][3 + S] : bs[S][f];
+          for (int f = 0; f < NF; ++f) b0[f] = T.baseIn ? win[f][3 + S] : bs[BSA ? S : 0][f];
           rk_store<C, EMIT>(a, T, o3, F, b0);
           if (a.pout) *(float *)((char *)a.pout + o3) = pp[S + 1];
         }
       }
-    } else {
-#pragma unroll
-      for (int f = 0; f < NF; ++f) gz[S + 1][f] = gz[S][f];
     }
     __syncthreads();
   };
 
   for (int it = it0; it < ze + 2; it += 2) {
     step(std::integral_constant<int, 0>{}, it);
-    if (it + 1 < ze + 2) step(std::integral_constant<int, 1>{}, it + 1);
+    if (it + 1 >= ze + 2) break;
+    step(std::integral_constant<int, 1>{}, it + 1);
     /* ---- rotate the carried arrays by two slots ---- */
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
@@ -1665,8 +1772,8 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
       for (int j = 0; j < 7; ++j) win[f][j] = win[f][j + 2];
       hv[0][f] = hv[2][f];
       hv[1][f] = hv[3][f];
-      bs[0][f] = bs[2][f];
-      gz[0][f] = gz[2][f];
+      if constexpr (BSA) bs[0][f] = bs[2][f];
+      if constexpr (FXR) fx[0][f] = fx[2][f];
     }
     pp[0] = pp[2]; pp[1] = pp[3]; pp[2] = pp[4];
     ri[0] = ri[2]; ri[1] = ri[3];
