@@ -24,6 +24,7 @@ namespace {
 constexpr long OW1 = OW1_, OB1 = OB1_, OW2 = OW2_, OB2 = OB2_, OW3 = OW3_, OB3 = OB3_, OW4 = OW4_, OB4 = OB4_,
                NPARAM = NPARAM_;
 constexpr long SGS_CHUNK = 262144;   /* cells per inference chunk */
+constexpr int GSPLIT = 64, GSPLIT_MIN = 128;   /* parts of a weight gradient, rows of the smallest (gemm_dw) */
 
 struct Sgs {
   float *w = nullptr, *gw = nullptr, *am = nullptr, *av = nullptr;
@@ -43,6 +44,7 @@ struct Sgs {
   long rows_cap = 0;
   float *Xb = nullptr, *Tb = nullptr, *Z[3] = {nullptr, nullptr, nullptr}, *Aa[3] = {nullptr, nullptr, nullptr};
   float *Y = nullptr, *dY = nullptr, *dA0 = nullptr, *dA1 = nullptr;
+  float *part = nullptr;                                                   /* partial weight gradients (gemm_dw) */
   int *idx = nullptr;
   long idx_cap = 0;
   double *dloss = nullptr;
@@ -88,65 +90,80 @@ int sgs_params_alloc() {
     HIPCHK(hipMemset(*q, 0, SGS_KIN * sizeof(float)));
   }
   if (!G.dloss) HIPCHK(hipMalloc(&G.dloss, sizeof(double)));
+  if (!G.part) HIPCHK(hipMalloc(&G.part, (size_t)GSPLIT * ((size_t)SGS_KIN * SGS_H + SGS_H) * sizeof(float)));
   return FE_OK;
 }
 
 hipStream_t sgs_stream() { return D.stream; }
+inline dim3 blocks(long n) { return dim3((unsigned)((n + 255) / 256)); }
 
-int gemm(const float *A, long sam, long sak, const float *B, long sbk, long sbn, float *C, long ldc, long M, int N, int K) {
-  if (M <= 0) return FE_OK;
-  GemmArgs g{A, sam, sak, B, sbk, sbn, C, ldc, (int)M, N, K};
-  dim3 grid((unsigned)((M + GT - 1) / GT), (unsigned)((N + GT - 1) / GT));
+/* C = A B with the epilogue of g (its epi, bias, act, Z) */
+int gemm(GemmArgs g) {
+  if (g.M <= 0) return FE_OK;
+  g.kchunk = (g.K + GK - 1) / GK * GK;
+  dim3 grid((unsigned)((g.M + GT - 1) / GT), (unsigned)((g.N + GT - 1) / GT));
   hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, sgs_stream(), g);
   HIPCHK(hipGetLastError());
   return FE_OK;
 }
 
-inline dim3 blocks(long n) { return dim3((unsigned)((n + 255) / 256)); }
+/* Gradient of a layer's weights [nin][nout] and, after them, biases [nout] into out:
+ * in^T dZ and the column sums of dZ over M rows.  Split over the rows into at most GSPLIT
+ * work-groups per output tile of at least 128 rows each (four K steps: below that the partial
+ * sums cost more than the steps they replace); 8192 rows: 64 parts, one part 1350 us. */
+int gemm_dw(const float *in, int nin, const float *dZ, int nout, long M, float *out) {
+  GemmArgs g{in, 1, nin, dZ, nout, 1, out, nout, nin, nout, (int)M};
+  const long n = (long)nin * nout + nout;
+  const long chunk = std::max<long>(GSPLIT_MIN, (M + GSPLIT - 1) / GSPLIT);
+  g.kchunk = (int)((chunk + GK - 1) / GK * GK);
+  const int nz = (int)((M + g.kchunk - 1) / g.kchunk);
+  if (nz > 1) { g.C = G.part; g.zstride = n; }
+  g.csum = g.C + (long)nin * nout;
+  dim3 grid((unsigned)((nin + GT - 1) / GT), (unsigned)((nout + GT - 1) / GT), (unsigned)nz);
+  hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, sgs_stream(), g);
+  if (nz > 1) hipLaunchKernelGGL(k_gemm_reduce, blocks(n), dim3(256), 0, sgs_stream(), (const float *)G.part, nz, n, out);
+  HIPCHK(hipGetLastError());
+  return FE_OK;
+}
 
 /* forward of M rows of X (normalised features) into G.Y; activations kept in G.Z/G.Aa */
 int mlp_forward(const float *X, long M) {
   int rc;
-  hipStream_t s = sgs_stream();
   const float *in = X;
-  long ld = SGS_KIN;
   int K = SGS_KIN;
   const long ow[3] = {OW1, OW2, OW3}, ob[3] = {OB1, OB2, OB3};
   for (int l = 0; l < 3; ++l) {
-    if ((rc = gemm(in, ld, 1, G.w + ow[l], SGS_H, 1, G.Z[l], SGS_H, M, SGS_H, K))) return rc;
-    hipLaunchKernelGGL(k_bias_act, blocks(M * SGS_H), dim3(256), 0, s, G.Z[l], G.Aa[l], (const float *)(G.w + ob[l]), M, SGS_H, 1);
+    GemmArgs g{in, K, 1, G.w + ow[l], SGS_H, 1, G.Z[l], SGS_H, (int)M, SGS_H, K};
+    g.epi = GEMM_BIAS_GELU; g.bias = G.w + ob[l]; g.act = G.Aa[l];
+    if ((rc = gemm(g))) return rc;
     in = G.Aa[l];
-    ld = SGS_H;
     K = SGS_H;
   }
-  if ((rc = gemm(in, SGS_H, 1, G.w + OW4, SGS_KOUT, 1, G.Y, SGS_KOUT, M, SGS_KOUT, SGS_H))) return rc;
-  hipLaunchKernelGGL(k_bias_act, blocks(M * SGS_KOUT), dim3(256), 0, s, G.Y, G.Y, (const float *)(G.w + OB4), M, SGS_KOUT, 0);
-  HIPCHK(hipGetLastError());
-  return FE_OK;
+  GemmArgs g{in, SGS_H, 1, G.w + OW4, SGS_KOUT, 1, G.Y, SGS_KOUT, (int)M, SGS_KOUT, SGS_H};
+  g.epi = GEMM_BIAS; g.bias = G.w + OB4;
+  return gemm(g);
 }
 
 /* backward of the loss gradient G.dY (M rows) into G.gw */
 int mlp_backward(const float *X, long M) {
   int rc;
-  hipStream_t s = sgs_stream();
   /* output layer */
-  if ((rc = gemm(G.Aa[2], 1, SGS_H, G.dY, SGS_KOUT, 1, G.gw + OW4, SGS_KOUT, SGS_H, SGS_KOUT, (int)M))) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(SGS_KOUT), dim3(256), 0, s, (const float *)G.dY, M, SGS_KOUT, G.gw + OB4);
-  if ((rc = gemm(G.dY, SGS_KOUT, 1, G.w + OW4, 1, SGS_KOUT, G.dA0, SGS_H, M, SGS_H, SGS_KOUT))) return rc;
-  const long ow[3] = {OW1, OW2, OW3}, ob[3] = {OB1, OB2, OB3};
-  float *dA = G.dA0, *dAn = G.dA1;
+  if ((rc = gemm_dw(G.Aa[2], SGS_H, G.dY, SGS_KOUT, M, G.gw + OW4))) return rc;
+  const long ow[3] = {OW1, OW2, OW3};
+  const float *dY = G.dY, *w = G.w + OW4;
+  int nout = SGS_KOUT;
+  float *dZ = G.dA0, *dZn = G.dA1;
   for (int l = 2; l >= 0; --l) {
-    hipLaunchKernelGGL(k_act_back, blocks(M * SGS_H), dim3(256), 0, s, (const float *)G.Z[l], dA, M * SGS_H);
-    const float *in = l > 0 ? G.Aa[l - 1] : X;
-    const int nin = l > 0 ? SGS_H : SGS_KIN;
-    if ((rc = gemm(in, 1, nin, dA, SGS_H, 1, G.gw + ow[l], SGS_H, nin, SGS_H, (int)M))) return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(SGS_H), dim3(256), 0, s, (const float *)dA, M, SGS_H, G.gw + ob[l]);
-    if (l > 0) {
-      if ((rc = gemm(dA, SGS_H, 1, G.w + ow[l], 1, SGS_H, dAn, SGS_H, M, SGS_H, SGS_H))) return rc;
-      std::swap(dA, dAn);
-    }
+    /* dZ of layer l: (dY W^T) GELU'(Z) */
+    GemmArgs g{dY, nout, 1, w, 1, nout, dZ, SGS_H, (int)M, SGS_H, nout};
+    g.epi = GEMM_GELU_BACK; g.Z = G.Z[l];
+    if ((rc = gemm(g))) return rc;
+    if ((rc = gemm_dw(l > 0 ? G.Aa[l - 1] : X, l > 0 ? SGS_H : SGS_KIN, dZ, SGS_H, M, G.gw + ow[l]))) return rc;
+    dY = dZ;
+    w = G.w + ow[l];
+    nout = SGS_H;
+    std::swap(dZ, dZn);
   }
-  HIPCHK(hipGetLastError());
   return FE_OK;
 }
 
@@ -211,7 +228,7 @@ int sgs_correct(float *Sout, float coefdt) {
 int sgs_free_all() {
   float **p[] = {&G.w, &G.gw, &G.am, &G.av, &G.xmu, &G.xisd, &G.ymu, &G.ysd, &G.Xs, &G.Ts, &G.Sc, &G.j33c, &G.Xb, &G.Tb,
                  &G.Z[0], &G.Z[1], &G.Z[2], &G.Aa[0], &G.Aa[1], &G.Aa[2], &G.Y, &G.dY, &G.dA0, &G.dA1, &G.tauL, &G.gmax, &G.j33,
-                 &G.grad, &G.Tf};
+                 &G.grad, &G.Tf, &G.part};
   if (D.stream) HIPCHK(hipStreamSynchronize(D.stream));
   for (auto q : p) if (*q) { HIPCHK(hipFree(*q)); *q = nullptr; }
   if (G.idx) HIPCHK(hipFree(G.idx));

@@ -32,64 +32,120 @@ constexpr long OW1_ = 0, OB1_ = OW1_ + (long)SGS_KIN * SGS_H, OW2_ = OB1_ + SGS_
 /* FP32 -> BF16, round to nearest even (the hardware conversion, v_cvt_pk_bf16_f32) */
 __device__ __forceinline__ unsigned short f2bf(float f) { return __builtin_bit_cast(unsigned short, (__bf16)f); }
 
+enum { GEMM_PLAIN = 0, GEMM_BIAS, GEMM_BIAS_GELU, GEMM_GELU_BACK };
+
 struct GemmArgs {
-  const float *A; long sam, sak;   /* A(m, k) = A[m*sam + k*sak] */
-  const float *B; long sbk, sbn;   /* B(k, n) = B[k*sbk + n*sbn] */
+  const float *A; long sam, sak;   /* A(m, k) = A[m*sam + k*sak], one of the strides 1 */
+  const float *B; long sbk, sbn;   /* B(k, n) = B[k*sbk + n*sbn], one of the strides 1 */
   float *C; long ldc;              /* C(m, n) = C[m*ldc + n] */
   int M, N, K;
+  int kchunk;                      /* rows of k per work-group z (a multiple of GK) */
+  long zstride;                    /* C (and csum) of work-group z start z*zstride further on */
+  float *csum;                     /* sum over k of B(k, n) in FP32 (null: none; needs sbn = 1) */
+  int epi;                         /* GEMM_*: what is applied to the product */
+  const float *bias;               /* GEMM_BIAS*: C = A B + bias (row broadcast) */
+  float *act;                      /* GEMM_BIAS_GELU: GELU(C), same layout as C */
+  const float *Z;                  /* GEMM_GELU_BACK: C = (A B) GELU'(Z), same layout as C */
 };
 
 constexpr int GT = 64, GK = 32, GKP = GK + 4;
+
+/* GELU and its derivative (below) */
+__device__ __forceinline__ float gelu(float z);
+__device__ __forceinline__ float gelu_d(float z);
+
+/* Four consecutive values of an operand tile: element (r, c) at p + r*ld + c, c the unit-stride
+ * index; columns at or past nc and rows at or past nr are 0.  vec: 16-byte loads are aligned. */
+__device__ __forceinline__ f32x4 tile4(const float *p, long ld, long r, long c, long nr, long nc, bool vec) {
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (r < nr) {
+    const float *q = p + r * ld + c;
+    if (vec && c + 3 < nc) v = *(const f32x4 *)q;
+    else
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c + i < nc) v[i] = q[i];
+  }
+  return v;
+}
 
 /* C = A B on 64 x 64 output tiles, four waves of 32 x 32, v_mfma_f32_16x16x16_bf16 over
  * K steps of 32 staged in LDS (k contiguous per row and per column, so each lane's four
  * operand values are adjacent).  Operand layout of the instruction: lane l holds
  * A[l % 16][4 (l / 16) + v] and B[4 (l / 16) + v][l % 16], v = 0..3, and receives
- * D[4 (l / 16) + v][l % 16]. */
+ * D[4 (l / 16) + v][l % 16].
+ * The network's products are small: what bounds them is the latency of a K step (load, stage,
+ * multiply) and the launches around them.  So the next step's operands are loaded (16 bytes per
+ * lane where alignment allows) before the current step is multiplied, LDS has two buffers (one
+ * barrier per step), bias, GELU and GELU' are applied to the accumulators instead of in passes of
+ * their own, and a product over the rows of a batch (the weight gradients: 64 or 256 x 64 outputs,
+ * thousands of k) is split over k into work-groups whose partial sums k_gemm_reduce adds in order;
+ * the bias gradient is the column sum of B, formed from the same loads.  8192 rows, forward and
+ * backward: first layer 50 -> 21 us, a weight gradient 1350 us (1 or 4 work-groups) -> 14 us. */
 __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
-  __shared__ unsigned short As[GT][GKP];
-  __shared__ unsigned short Bs[GT][GKP];
+  __shared__ __align__(16) unsigned short As[2][GT][GKP];
+  __shared__ __align__(16) unsigned short Bs[2][GT][GKP];
+  __shared__ __align__(16) float cs[16][GT];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int m0 = blockIdx.x * GT, n0 = blockIdx.y * GT;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  const int kbeg = blockIdx.z * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
+  float *C = g.C + (long)blockIdx.z * g.zstride;
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const bool a_krow = (g.sak == 1), b_ncol = (g.sbn == 1);
-  for (int k0 = 0; k0 < g.K; k0 += GK) {
-    for (int e = tid; e < GT * GK; e += 256) {
-      int mm, kk;
-      if (a_krow) { mm = e / GK; kk = e % GK; } else { kk = e / GT; mm = e % GT; }
-      const int m = m0 + mm, k = k0 + kk;
-      const float v = (m < g.M && k < g.K) ? g.A[(long)m * g.sam + (long)k * g.sak] : 0.f;
-      As[mm][kk] = f2bf(v);
+  const long lda = a_krow ? g.sam : g.sak, ldb = b_ncol ? g.sbk : g.sbn;
+  const bool va = ((unsigned long)g.A & 15) == 0 && (lda & 3) == 0, vb = ((unsigned long)g.B & 15) == 0 && (ldb & 3) == 0;
+  /* element e of a tile, four values wide: (row e / 8, k 4 (e % 8)) where k is the unit-stride
+   * index, (k e / 16, row 4 (e % 16)) where the row is */
+  auto loads = [&](int k0, f32x4 (&ra)[2], f32x4 (&rb)[2]) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int e = tid + 256 * q;
+      ra[q] = a_krow ? tile4(g.A, lda, m0 + (e >> 3), k0 + 4 * (e & 7), g.M, kend, va)
+                     : tile4(g.A, lda, k0 + (e >> 4), m0 + 4 * (e & 15), kend, g.M, va);
+      rb[q] = b_ncol ? tile4(g.B, ldb, k0 + (e >> 4), n0 + 4 * (e & 15), kend, g.N, vb)
+                     : tile4(g.B, ldb, n0 + (e >> 3), k0 + 4 * (e & 7), g.N, kend, vb);
     }
-    for (int e = tid; e < GT * GK; e += 256) {
-      int nn, kk;
-      if (b_ncol) { kk = e / GT; nn = e % GT; } else { nn = e / GK; kk = e % GK; }
-      const int n = n0 + nn, k = k0 + kk;
-      const float v = (n < g.N && k < g.K) ? g.B[(long)k * g.sbk + (long)n * g.sbn] : 0.f;
-      Bs[nn][kk] = f2bf(v);
+  };
+  auto stage = [&](unsigned short (*T)[GKP], const f32x4 &v, int e, bool krow) {
+    if (krow) {
+      *(bf16x4 *)&T[e >> 3][4 * (e & 7)] = bf16x4{(short)f2bf(v[0]), (short)f2bf(v[1]), (short)f2bf(v[2]), (short)f2bf(v[3])};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) T[4 * (e & 15) + i][e >> 4] = f2bf(v[i]);
     }
+  };
+  const bool do_cs = g.csum && blockIdx.x == 0;
+  f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 ra[2], rb[2];
+  loads(kbeg, ra, rb);
+  int buf = 0;
+  for (int k0 = kbeg; k0 < kend; k0 += GK, buf ^= 1) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      stage(As[buf], ra[q], tid + 256 * q, a_krow);
+      stage(Bs[buf], rb[q], tid + 256 * q, !b_ncol);
+      if (do_cs) sum += rb[q];
+    }
+    if (k0 + GK < kend) loads(k0 + GK, ra, rb);
     __syncthreads();
 #pragma unroll
     for (int ks = 0; ks < GK; ks += 16) {
       bf16x4 a[2], b[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const unsigned short *pa = &As[wm + 16 * i + (lane & 15)][ks + 4 * (lane >> 4)];
-        const unsigned short *pb = &Bs[wn + 16 * i + (lane & 15)][ks + 4 * (lane >> 4)];
-        a[i] = bf16x4{(short)pa[0], (short)pa[1], (short)pa[2], (short)pa[3]};
-        b[i] = bf16x4{(short)pb[0], (short)pb[1], (short)pb[2], (short)pb[3]};
+        a[i] = *(const bf16x4 *)&As[buf][wm + 16 * i + (lane & 15)][ks + 4 * (lane >> 4)];
+        b[i] = *(const bf16x4 *)&Bs[buf][wn + 16 * i + (lane & 15)][ks + 4 * (lane >> 4)];
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -98,8 +154,35 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int m = m0 + wm + 16 * i + 4 * (lane >> 4) + v, n = n0 + wn + 16 * j + (lane & 15);
-        if (m < g.M && n < g.N) g.C[(long)m * g.ldc + n] = acc[i][j][v];
+        if (m < g.M && n < g.N) {
+          const long o = (long)m * g.ldc + n;
+          float c = acc[i][j][v];
+          if (g.epi == GEMM_BIAS || g.epi == GEMM_BIAS_GELU) c = c + g.bias[n];
+          if (g.epi == GEMM_GELU_BACK) c = c * gelu_d(g.Z[o]);
+          C[o] = c;
+          if (g.epi == GEMM_BIAS_GELU) g.act[o] = gelu(c);
+        }
       }
+  if (do_cs) {                     /* uniform over the work-group */
+    *(f32x4 *)&cs[tid >> 4][4 * (tid & 15)] = sum;
+    __syncthreads();
+    if (tid < GT && n0 + tid < g.N) {
+      float t = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t += cs[r][tid];
+      g.csum[(long)blockIdx.z * g.zstride + n0 + tid] = t;
+    }
+  }
+}
+
+/* out[i] = sum over z of part[z*n + i], in order of z */
+__global__ void __launch_bounds__(256) k_gemm_reduce(const float *part, int nz, long n, float *out) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  float s = 0.f;
+#pragma unroll 8
+  for (int z = 0; z < nz; ++z) s += part[(long)z * n + i];
+  out[i] = s;
 }
 
 /* GELU(z) = z Phi(z) without transcendentals: Phi(z) = 1/2 + zc Q(zc^2), zc = z clamped to
@@ -136,33 +219,6 @@ __device__ __forceinline__ float gelu_d(float z) {
   return fmaf(zc, gelu_q(s), 0.5f) + (fabsf(z) < 4.f ? z * d : 0.f);
 }
 
-/* Z += b (row broadcast); A = GELU(Z) (act) or Z */
-__global__ void k_bias_act(float *Z, float *A, const float *b, long M, int N, int act) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M * N) return;
-  const float z = Z[i] + b[i % N];
-  Z[i] = z;
-  A[i] = act ? gelu(z) : z;
-}
-
-/* dZ = dA * GELU'(Z), in place over dA */
-__global__ void k_act_back(const float *Z, float *dA, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dA[i] *= gelu_d(Z[i]);
-}
-
-/* db[n] = sum over rows of dZ[m][n]: one work-group per column */
-__global__ void __launch_bounds__(256) k_colsum(const float *dZ, long M, int N, float *db) {
-  const int n = blockIdx.x;
-  float s = 0.f;
-  for (long m = threadIdx.x; m < M; m += 256) s += dZ[m * N + n];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  __shared__ float part[4];
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) db[n] = (part[0] + part[1]) + (part[2] + part[3]);
-}
-
 /* mean-squared-error gradient over the first nout of N columns: dY = 2 (Y - T) / (M nout);
  * the loss sum (FP64) goes to loss[0] */
 __global__ void __launch_bounds__(256) k_loss_grad(const float *Y, const float *T, long M, int N, int nout, float *dY,
@@ -176,7 +232,13 @@ __global__ void __launch_bounds__(256) k_loss_grad(const float *Y, const float *
     l = (double)d * d;
   }
   for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-  if ((threadIdx.x & 63) == 0 && l != 0.0) atomicAdd(loss, l);
+  __shared__ double part[4];       /* one atomic per work-group: they queue up on the one address */
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = l;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    l = (part[0] + part[1]) + (part[2] + part[3]);
+    if (l != 0.0) atomicAdd(loss, l);
+  }
 }
 
 /* Adam (Kingma & Ba 2015) on FP32 master weights; bc1, bc2 = 1 - beta^t */
