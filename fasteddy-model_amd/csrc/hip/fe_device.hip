@@ -81,6 +81,9 @@ struct Dev {
   int nseg = 1, zseg = 0;          /* z segments of the stage launches and their length */
   float *lsfM = nullptr;           /* slab means of rho, rho*u, rho*v, rho*theta, rho*q_v, levels -1..Nz */
   float *lsfR = nullptr;           /* large-scale forcing rows, LSF_ROW per level */
+  double *lsfP = nullptr;          /* partial slab sums, [part][level -1..Nz][5] */
+  double *stat = nullptr;          /* workspace of the statistics reductions, kept from call to call */
+  size_t stat_n = 0;
   bool lsfNow = false;             /* the current step's last stage carries the forcing */
   long fs = 0, ps = 0;
   int np = 0;
@@ -480,41 +483,83 @@ int launch_stage(int stage, const float *in, const float *base, float *out, int 
   return FE_OK;
 }
 
-/* Slab means over the halo-inclusive plane (fecuda_PlugIns.cu:25-45 reduces the
- * halo-inclusive extents and divides by their product), one work-group per level
- * -1..Nz; halo values follow the boundary rules of the state (periodic sides; at the
- * bottom and lid: rho, rho*theta from the base state, rho*u, rho*v zero-gradient below
- * and geostrophic above, q_v zero-gradient).  FP64 sums. */
-__global__ void __launch_bounds__(256) k_lsf_means(const float *S, long fs, long ps, int Nx, int Ny, int Nz, int P, int Nh,
-                                                   int iqv, const float *prof, float uTop, float vTop, float *M) {
-  const int z = (int)blockIdx.x - 1;
-  const int nxh = Nx + 2 * Nh, nyh = Ny + 2 * Nh;
-  double acc[5] = {0, 0, 0, 0, 0};
-  for (int c = threadIdx.x; c < nxh * nyh; c += 256) {
-    const int j = c / nxh, i = c - j * nxh;
-    const int x = ((i - Nh) % Nx + Nx) % Nx, y = ((j - Nh) % Ny + Ny) % Ny;
-    const long col = (long)y * P + x;
-    const int zc = z < 0 ? 0 : (z >= Nz ? Nz - 1 : z);
-    const long o = (long)zc * ps + col;
-    const bool in = (z >= 0 && z < Nz);
-    acc[0] += in ? S[o] : prof[(z + 3) * PROW + PR_RHO];
-    acc[1] += in || z < 0 ? S[fs + o] : uTop;
-    acc[2] += in || z < 0 ? S[2 * fs + o] : vTop;
-    acc[3] += in ? S[4 * fs + o] : prof[(z + 3) * PROW + PR_RTH];
-    if (iqv >= 0) acc[4] += S[(long)iqv * fs + o];     /* iqv < 0: no q_v field */
-  }
+/* Work-groups per level of a plane reduction over n4 groups of four cells: about 1024 in all (four
+ * per compute unit, which keeps enough loads in flight for the copy rate; one per level left most
+ * of the chip idle and ran at the latency of one wave's loads), at least 256 groups each, at most
+ * `most`. */
+constexpr int STAT_NT = 256;
+static int stat_parts(int nlev, long n4, long most) {
+  return (int)std::max<long>(1, std::min<long>({(1024 + nlev - 1) / nlev, n4 / STAT_NT, most}));
+}
+
+/* Sums each of v[0..N) over the work-group's STAT_NT threads; thread k < N returns its total in v[0]. */
+template <int N, typename T>
+__device__ __forceinline__ void block_sums(T (&v)[N], T (*part)[N]) {
 #pragma unroll
-  for (int f = 0; f < 5; ++f)
-    for (int off = 32; off > 0; off >>= 1) acc[f] += __shfl_xor(acc[f], off);
-  __shared__ double part[4][5];
+  for (int k = 0; k < N; ++k)
+    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off);
   if (threadIdx.x % 64 == 0)
-    for (int f = 0; f < 5; ++f) part[threadIdx.x / 64][f] = acc[f];
+#pragma unroll
+    for (int k = 0; k < N; ++k) part[threadIdx.x / 64][k] = v[k];
   __syncthreads();
-  if (threadIdx.x < 5) {
-    const int f = threadIdx.x;
-    const double s = part[0][f] + part[1][f] + part[2][f] + part[3][f];
-    M[f * (Nz + 2) + z + 1] = (float)(s / ((double)nxh * (double)nyh));
+  if (threadIdx.x < N) {
+    T t = part[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < STAT_NT / 64; ++w) t += part[w][threadIdx.x];
+    v[0] = t;
   }
+}
+
+/* Slab means over the halo-inclusive plane (fecuda_PlugIns.cu:25-45 reduces the
+ * halo-inclusive extents and divides by their product), levels -1..Nz; halo values follow the
+ * boundary rules of the state (periodic sides: a column counts as often as the halo-inclusive
+ * plane holds its images; at the bottom and lid: rho, rho*theta from the base state, rho*u, rho*v
+ * zero-gradient below and geostrophic above, q_v zero-gradient).  FP64 sums of work-group
+ * (part, level) into part, [part][level][5]; k_lsf_mean adds the parts in order.  Bound by the
+ * loads of five fields: 152 x 146 x 122, one work-group per level 113 us, parts 19 us. */
+__global__ void __launch_bounds__(STAT_NT) k_lsf_sums(const float *S, long fs, long ps, int Nx, int Ny, int Nz, int P, int Nh,
+                                                      int iqv, const float *prof, float uTop, float vTop, long chunk,
+                                                      double *out) {
+  const int z = (int)blockIdx.x - 1;
+  const int g = (Nx + 3) / 4;
+  const long n4 = (long)g * Ny, i1 = min(n4, (long)(blockIdx.y + 1) * chunk);
+  /* halo-inclusive positions -Nh .. N+Nh-1 that wrap to v */
+  auto images = [&](int v, int N) { return (N + Nh - 1 - v) / N + (v + Nh) / N + 1; };
+  const int zc = z < 0 ? 0 : (z >= Nz ? Nz - 1 : z);
+  const bool in = (z >= 0 && z < Nz);
+  const float r0 = prof[(z + 3) * PROW + PR_RHO], t0 = prof[(z + 3) * PROW + PR_RTH];
+  double acc[5] = {0, 0, 0, 0, 0};
+  for (long i = (long)blockIdx.y * chunk + threadIdx.x; i < i1; i += STAT_NT) {
+    const int y = (int)(i / g), x = 4 * (int)(i - (long)y * g);
+    const long o = (long)zc * ps + (long)y * P + x;
+    const float4 a = *(const float4 *)(S + o), b = *(const float4 *)(S + fs + o), c = *(const float4 *)(S + 2 * fs + o),
+                 d = *(const float4 *)(S + 4 * fs + o);
+    const float4 q = iqv >= 0 ? *(const float4 *)(S + (long)iqv * fs + o) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float va[4] = {a.x, a.y, a.z, a.w}, vb[4] = {b.x, b.y, b.z, b.w}, vc[4] = {c.x, c.y, c.z, c.w},
+                vd[4] = {d.x, d.y, d.z, d.w}, vq[4] = {q.x, q.y, q.z, q.w};
+    const double wy = images(y, Ny);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (x + j >= Nx) continue;                     /* the row's padding */
+      const double w = wy * images(x + j, Nx);
+      acc[0] += w * (in ? va[j] : r0);
+      acc[1] += w * (in || z < 0 ? vb[j] : uTop);
+      acc[2] += w * (in || z < 0 ? vc[j] : vTop);
+      acc[3] += w * (in ? vd[j] : t0);
+      acc[4] += w * vq[j];                           /* iqv < 0: no q_v field */
+    }
+  }
+  __shared__ double part[STAT_NT / 64][5];
+  block_sums(acc, part);
+  if (threadIdx.x < 5) out[((long)blockIdx.y * (Nz + 2) + blockIdx.x) * 5 + threadIdx.x] = acc[0];
+}
+__global__ void k_lsf_mean(const double *part, int parts, int nlev, double cells, float *M) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;   /* (level, field) */
+  if (i >= nlev * 5) return;
+  double s = 0.0;
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p) s += part[(long)p * nlev * 5 + i];
+  M[(i % 5) * nlev + i / 5] = (float)(s / cells);
 }
 
 struct LsfPar { float p[3][5]; int horMn, moist; float fac; };
@@ -573,8 +618,12 @@ int lsf_prepare() {
   const int itn = (int)roundf(lsf_freq / dt);
   if (!(simTime_it > simTime_itRestart && itn > 0 && simTime_it % itn == 0)) return FE_OK;
   if (lsf_horMnSubTerms == 1) {
-    hipLaunchKernelGGL(k_lsf_means, dim3(D.Nz + 2), dim3(256), 0, D.stream, D.S[0], D.fs, D.ps, D.Nx, D.Ny, D.Nz, D.P, D.Nh,
-                       D.nM > 0 ? 5 + D.nTKE : -1, D.prof, D.uTop, D.vTop, D.lsfM);
+    const long n4 = (long)((D.Nx + 3) / 4) * D.Ny;
+    const int parts = stat_parts(D.Nz + 2, n4, LONG_MAX);
+    hipLaunchKernelGGL(k_lsf_sums, dim3(D.Nz + 2, parts), dim3(STAT_NT), 0, D.stream, D.S[0], D.fs, D.ps, D.Nx, D.Ny, D.Nz, D.P,
+                       D.Nh, D.nM > 0 ? 5 + D.nTKE : -1, D.prof, D.uTop, D.vTop, (n4 + parts - 1) / parts, D.lsfP);
+    hipLaunchKernelGGL(k_lsf_mean, dim3((5 * (D.Nz + 2) + 63) / 64), dim3(64), 0, D.stream, (const double *)D.lsfP, parts, D.Nz + 2,
+                       (double)(D.Nx + 2 * D.Nh) * (double)(D.Ny + 2 * D.Nh), D.lsfM);
     HIPCHK(hipGetLastError());
   }
   if (simTime_it - simTime_itRestart < itn) return FE_OK;
@@ -1028,6 +1077,7 @@ int cuda_hydroCoreInit(void) {
   if (lsfSelector == 1) {
     HIPCHK(hipMalloc(&D.lsfM, (size_t)5 * (D.Nz + 2) * sizeof(float)));
     HIPCHK(hipMemset(D.lsfM, 0, (size_t)5 * (D.Nz + 2) * sizeof(float)));
+    HIPCHK(hipMalloc(&D.lsfP, (size_t)stat_parts(D.Nz + 2, (long)((D.Nx + 3) / 4) * D.Ny, LONG_MAX) * (D.Nz + 2) * 5 * sizeof(double)));
     HIPCHK(hipMalloc(&D.lsfR, (size_t)LSF_ROW * D.Nz * sizeof(float)));
     HIPCHK(hipMemset(D.lsfR, 0, (size_t)LSF_ROW * D.Nz * sizeof(float)));
   }
@@ -1039,6 +1089,9 @@ int cuda_hydroCoreCleanup(void) {
   for (int s = 0; s < 3; ++s) if (D.S[s]) { (void)hipFree(D.S[s]); D.S[s] = nullptr; }
   float **p[] = {&D.pout, &D.tau, &D.mtau, &D.fem, &D.surf, &D.stg, &D.lsfM, &D.lsfR, &D.tprof};
   for (auto q : p) if (*q) { (void)hipFree(*q); *q = nullptr; }
+  double **pd[] = {&D.lsfP, &D.stat};
+  for (auto q : pd) if (*q) { (void)hipFree(*q); *q = nullptr; }
+  D.stat_n = 0;
   D.hydro = 0;
   return FE_OK;
 }
@@ -1176,58 +1229,70 @@ double fe_copy_probe(long nfloats, int reps) {
 
 /* Horizontal-mean profile statistics of the device state in FP64, the on-device
  * counterpart of the reference's post-processing of an output state
- * (tutorials/notebooks/fetutorialfunctions.py:55-83,344-431).  One work-group per
- * level accumulates the level sums of u, v, w, theta (rho-weighted fields over
- * rho), their products, and the SGS TKE and moisture per unit mass; each
- * wavefront reduces its lanes with cross-lane shuffles, and the wavefronts'
- * partial sums meet in LDS.  Output columns, per level:
+ * (tutorials/notebooks/fetutorialfunctions.py:55-83,344-431).  The work-groups of a
+ * level accumulate the sums of u, v, w, theta (rho-weighted fields over
+ * rho), their products, and the SGS TKE and moisture per unit mass over their
+ * part of its cells, four cells per thread and load; each
+ * wavefront reduces its lanes with cross-lane shuffles, the wavefronts'
+ * partial sums meet in LDS, and k_profiles_final adds a level's parts in order.
+ * 256 x 256 x 96, eight fields (201 MB): one work-group per level 324 us, parts 52 us.
+ * Output columns, per level:
  *   0 <u> 1 <v> 2 <w> 3 <theta> 4 <u'u'> 5 <u'w'> 6 <v'v'> 7 <v'w'> 8 <w'w'>
  *   9 resolved TKE 10 <theta'w'> 11 <e> 12 <q_v> 13 <q_l>
  *   14 (<tau13>^2 + <tau23>^2)^1/2, 15 <tau33>, 16 <tau_theta3> (level means of the SGS
  *   stresses emitted by the last batch; moved to cell centres on the host)
  * (covariances from FP64 first and second moments). */
-constexpr int PROF_NSTAT = 17, PROF_NSUM = 17, PROF_NT = 256;
-__global__ void __launch_bounds__(PROF_NT) k_profiles(const float *S, long fs, long ps, int Nx, int Ny, int P, int nTKE,
-                                                      int nM, const float *tau, double *out) {
-  const int z = blockIdx.x;
+constexpr int PROF_NSTAT = 17, PROF_NSUM = 17;
+__global__ void __launch_bounds__(STAT_NT) k_profiles(const float *S, long fs, long ps, int Nx, int Ny, int P, int nTKE,
+                                                      int nM, const float *tau, long chunk, double *out) {
+  const int z = blockIdx.x, g = (Nx + 3) / 4;
+  const long n4 = (long)g * Ny, i1 = min(n4, (long)(blockIdx.y + 1) * chunk);
   double acc[PROF_NSUM];
 #pragma unroll
   for (int k = 0; k < PROF_NSUM; ++k) acc[k] = 0.0;
-  const int n = Nx * Ny;
-  for (int i = threadIdx.x; i < n; i += PROF_NT) {
-    const int y = i / Nx, x = i - y * Nx;
+  for (long i = (long)blockIdx.y * chunk + threadIdx.x; i < i1; i += STAT_NT) {
+    const int y = (int)(i / g), x = 4 * (int)(i - (long)y * g);
     const long o = (long)z * ps + (long)y * P + x;
-    const double rho = S[o];
-    const double u = S[fs + o] / rho, v = S[2 * fs + o] / rho, w = S[3 * fs + o] / rho, th = S[4 * fs + o] / rho;
-    acc[0] += u; acc[1] += v; acc[2] += w; acc[3] += th;
-    acc[4] += u * u; acc[5] += u * w; acc[6] += v * v; acc[7] += v * w; acc[8] += w * w; acc[9] += th * w;
-    if (nTKE > 0) acc[10] += S[5 * fs + o] / rho;
-    if (nM > 0) acc[11] += S[(long)(5 + nTKE) * fs + o] / rho;
-    if (nM > 1) acc[12] += S[(long)(6 + nTKE) * fs + o] / rho;
-    if (tau) {
-      acc[13] += tau[2 * fs + o];
-      acc[14] += tau[3 * fs + o];
-      acc[15] += tau[5 * fs + o];
-      acc[16] += tau[8 * fs + o];
+    /* rows are padded to whole 128-byte lines, so the last group of a row stays inside its row */
+    auto ld = [&](const float *p, float (&v)[4]) {
+      const float4 t = *(const float4 *)(p + o);
+      v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    };
+    float r[4], a[4], b[4], c[4], d[4], e[4] = {0.f, 0.f, 0.f, 0.f}, q[4] = {0.f, 0.f, 0.f, 0.f}, l[4] = {0.f, 0.f, 0.f, 0.f};
+    float t1[4] = {0.f, 0.f, 0.f, 0.f}, t2[4] = {0.f, 0.f, 0.f, 0.f}, t3[4] = {0.f, 0.f, 0.f, 0.f}, t4[4] = {0.f, 0.f, 0.f, 0.f};
+    ld(S, r); ld(S + fs, a); ld(S + 2 * fs, b); ld(S + 3 * fs, c); ld(S + 4 * fs, d);
+    if (nTKE > 0) ld(S + 5 * fs, e);
+    if (nM > 0) ld(S + (long)(5 + nTKE) * fs, q);
+    if (nM > 1) ld(S + (long)(6 + nTKE) * fs, l);
+    if (tau) { ld(tau + 2 * fs, t1); ld(tau + 3 * fs, t2); ld(tau + 5 * fs, t3); ld(tau + 8 * fs, t4); }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (x + j >= Nx) continue;
+      const double rho = r[j];
+      const double u = a[j] / rho, v = b[j] / rho, w = c[j] / rho, th = d[j] / rho;
+      acc[0] += u; acc[1] += v; acc[2] += w; acc[3] += th;
+      acc[4] += u * u; acc[5] += u * w; acc[6] += v * v; acc[7] += v * w; acc[8] += w * w; acc[9] += th * w;
+      if (nTKE > 0) acc[10] += e[j] / rho;
+      if (nM > 0) acc[11] += q[j] / rho;
+      if (nM > 1) acc[12] += l[j] / rho;
+      if (tau) { acc[13] += t1[j]; acc[14] += t2[j]; acc[15] += t3[j]; acc[16] += t4[j]; }
     }
   }
-#pragma unroll
-  for (int k = 0; k < PROF_NSUM; ++k)
-    for (int off = 32; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off);
-  __shared__ double part[PROF_NT / 64][PROF_NSUM];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < PROF_NSUM; ++k) part[wave][k] = acc[k];
+  __shared__ double part[STAT_NT / 64][PROF_NSUM];
+  block_sums(acc, part);
+  if (threadIdx.x < PROF_NSUM) out[((long)blockIdx.y * gridDim.x + z) * PROF_NSTAT + threadIdx.x] = acc[0];
+}
+/* Level z's sums over its parts, then its profile row, in place of part 0's row. */
+__global__ void __launch_bounds__(64) k_profiles_final(double *out, int parts, int nlev, double n) {
+  const int z = blockIdx.x, k = threadIdx.x;
+  __shared__ double s[PROF_NSUM];
+  if (k < PROF_NSUM) {
+    double t = 0.0;
+    for (int p = 0; p < parts; ++p) t += out[((long)p * nlev + z) * PROF_NSTAT + k];
+    s[k] = t / n;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double s[PROF_NSUM];
-    for (int k = 0; k < PROF_NSUM; ++k) {
-      s[k] = 0.0;
-      for (int wv = 0; wv < PROF_NT / 64; ++wv) s[k] += part[wv][k];
-      s[k] /= (double)n;
-    }
+  if (k == 0) {
     double *r = out + (long)z * PROF_NSTAT;
     r[0] = s[0]; r[1] = s[1]; r[2] = s[2]; r[3] = s[3];
     r[4] = s[4] - s[0] * s[0];
@@ -1274,27 +1339,48 @@ static void profiles_centre_sgs(double *out, int nz) {
   }
 }
 
+/* The profile rows of the current state into d[0 .. Nz), which has room for every part's rows:
+ * parts x Nz <= FE_NOALLOC_MAX_LEVELS (or one part), the same for both entry points, so that they
+ * give the same bits; then to out. */
+static int profiles_parts(void) {
+  return stat_parts(D.Nz, (long)((D.Nx + 3) / 4) * D.Ny, std::max(1, FE_NOALLOC_MAX_LEVELS / D.Nz));
+}
+static int profiles_run(double *d, double *out) {
+  const int parts = profiles_parts();
+  const long n4 = (long)((D.Nx + 3) / 4) * D.Ny;
+  hipLaunchKernelGGL(k_profiles, dim3(D.Nz, parts), dim3(STAT_NT), 0, D.stream, D.S[0], D.fs, D.ps, D.Nx, D.Ny, D.P, D.nTKE, D.nM,
+                     D.tau, (n4 + parts - 1) / parts, d);
+  hipLaunchKernelGGL(k_profiles_final, dim3(D.Nz), dim3(64), 0, D.stream, d, parts, D.Nz, (double)D.Nx * D.Ny);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(out, d, (size_t)D.Nz * PROF_NSTAT * sizeof(double), hipMemcpyDeviceToHost, D.stream));
+  HIPCHK(hipStreamSynchronize(D.stream));
+  profiles_centre_sgs(out, D.Nz);
+  return FE_OK;
+}
+
+/* n doubles of the model's statistics workspace (kept until cuda_hydroCoreCleanup) */
+static int stat_space(size_t n) {
+  if (n <= D.stat_n) return FE_OK;
+  if (D.stat) HIPCHK(hipFree(D.stat));
+  D.stat = nullptr;
+  D.stat_n = 0;
+  HIPCHK(hipMalloc(&D.stat, n * sizeof(double)));
+  D.stat_n = n;
+  return FE_OK;
+}
+
 int fe_profiles(double *out, int nstat) {
   if (!D.hydro) return FE_ERR_STATE;
   if (nstat != PROF_NSTAT || !out) return FE_ERR_UNSUPPORTED;
-  double *d = nullptr;
-  HIPCHK(hipMalloc(&d, (size_t)D.Nz * PROF_NSTAT * sizeof(double)));
-  hipLaunchKernelGGL(k_profiles, dim3(D.Nz), dim3(PROF_NT), 0, D.stream, D.S[0], D.fs, D.ps, D.Nx, D.Ny, D.P, D.nTKE, D.nM,
-                     D.tau, d);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(out, d, (size_t)D.Nz * PROF_NSTAT * sizeof(double), hipMemcpyDeviceToHost, D.stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(D.stream);
-  const hipError_t ef = hipFree(d);
-  if (e == hipSuccess) e = ef;
-  HIPCHK(e);
-  profiles_centre_sgs(out, D.Nz);
-  return FE_OK;
+  int rc;
+  if ((rc = stat_space((size_t)profiles_parts() * D.Nz * PROF_NSTAT))) return rc;
+  return profiles_run(D.stat, out);
 }
 
 /* fe_profiles without any device allocation: the per-level rows go to the library's
  * static scratch array (no hipMalloc/hipFree; the only device memory touched besides the
  * state is that array).  Grids of more than FE_NOALLOC_MAX_LEVELS levels are rejected.
- * Every row the kernel writes is written completely, so nothing needs clearing; calls
+ * Every row the kernels read they have written in the same call, so nothing needs clearing; calls
  * that overlap on one GPU share the array and race. */
 int fe_profiles_noalloc(double *out, int nstat) {
   if (!D.hydro) return FE_ERR_STATE;
@@ -1306,14 +1392,7 @@ int fe_profiles_noalloc(double *out, int nstat) {
   int rc, dev = 0;
   if ((rc = scratch_lookup())) return rc;
   HIPCHK(hipGetDevice(&dev));
-  double *d = g_scratch_ptr[dev];
-  hipLaunchKernelGGL(k_profiles, dim3(D.Nz), dim3(PROF_NT), 0, D.stream, D.S[0], D.fs, D.ps, D.Nx, D.Ny, D.P, D.nTKE, D.nM,
-                     D.tau, d);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(out, d, (size_t)D.Nz * PROF_NSTAT * sizeof(double), hipMemcpyDeviceToHost, D.stream));
-  HIPCHK(hipStreamSynchronize(D.stream));
-  profiles_centre_sgs(out, D.Nz);
-  return FE_OK;
+  return profiles_run(g_scratch_ptr[dev], out);
 }
 
 /* Per-field state summary of the device state, the on-device counterpart of the
@@ -1324,55 +1403,81 @@ int fe_profiles_noalloc(double *out, int nstat) {
  * rho, u, v, w, theta (rho-weighted fields times float(1/rho), as the reference
  * forms them), p', the SGS TKE and the moisture species per unit mass; plus the
  * horizontal sum of the raw (rho-weighted) field, from which the host forms its
- * volume integral (mass, rho*theta, ... budgets).  One work-group per level; the
- * FP64 sums and the (value, location) extremes are reduced with cross-lane
- * shuffles, then across the wavefronts in LDS; the host combines the levels. */
-constexpr int SUM_NT = 256, SUM_NCOL = 12, SUM_LV = 8, SUM_MAXF = 9;
-__device__ __forceinline__ void sum_pick(float &v, long long &k, float v2, long long k2, bool is_max) {
+ * volume integral (mass, rho*theta, ... budgets).  Several work-groups per level, four cells
+ * per thread and load; the FP64 sums and the (value, location) extremes are reduced with
+ * cross-lane shuffles, then across the wavefronts in LDS, then over the level's parts; the host
+ * combines the levels.  256 x 256 x 96, nine rows (226 MB): one work-group per level 1186 us,
+ * parts 165 us (an extremes-of-four fast path for finite cells measured 440 us: registers). */
+constexpr int SUM_NCOL = 12, SUM_LV = 8, SUM_MAXF = 9;
+constexpr unsigned SUM_NONE = 0xffffffffu;      /* no location (a plane has fewer columns: fields are below 4 GiB) */
+__device__ __forceinline__ void sum_pick(float &v, unsigned &k, float v2, unsigned k2, bool is_max) {
   const bool take = is_max ? (v2 > v || (v2 == v && k2 < k)) : (v2 < v || (v2 == v && k2 < k));
   if (take) { v = v2; k = k2; }
 }
-__global__ void __launch_bounds__(SUM_NT) k_summary(const float *S, const float *pres, long fs, long ps, int Nx, int Ny, int Nz,
-                                                     int P, int ns, int nTKE, double *out, const float *dcol) {
-  const int z = blockIdx.x;
+/* Joins n partial rows, stride doubles apart, into one at to (which may be the first of them). */
+__device__ __forceinline__ void summary_join(const double *q, long stride, int n, double *to) {
+  float vx = (float)q[0], vn = (float)q[2];
+  unsigned kx = (unsigned)q[1], kn = (unsigned)q[3];
+  double a4 = q[4], a5 = q[5], a6 = q[6], a7 = q[7];
+  for (int i = 1; i < n; ++i) {
+    const double *p = q + (long)i * stride;
+    sum_pick(vx, kx, (float)p[0], (unsigned)p[1], true);
+    sum_pick(vn, kn, (float)p[2], (unsigned)p[3], false);
+    a4 += p[4]; a5 += p[5]; a6 += p[6]; a7 += p[7];
+  }
+  to[0] = vx; to[1] = (double)kx; to[2] = vn; to[3] = (double)kn; to[4] = a4; to[5] = a5; to[6] = a6; to[7] = a7;
+}
+/* Partial rows of work-group (part, level): [part][level][row][SUM_LV] = max, its column x Ny + y,
+ * min, its column, sum of the finite values, NaN count, Inf count, sum of the raw field. */
+__global__ void __launch_bounds__(STAT_NT) k_summary(const float *S, const float *pres, long fs, long ps, int Nx, int Ny,
+                                                      int P, int ns, long chunk, double *out, const float *dcol) {
+  const int z = blockIdx.x, g = (Nx + 3) / 4;
+  const long n4 = (long)g * Ny, i1 = min(n4, (long)(blockIdx.y + 1) * chunk);
   float mx[SUM_MAXF], mn[SUM_MAXF];
-  long long kx[SUM_MAXF], kn[SUM_MAXF];
+  unsigned kx[SUM_MAXF], kn[SUM_MAXF], nnan[SUM_MAXF], ninf[SUM_MAXF];
   double sm[SUM_MAXF], raw[SUM_MAXF];
-  int nnan[SUM_MAXF], ninf[SUM_MAXF];
-  const long long NONE = 0x7fffffffffffffffLL;
 #pragma unroll
   for (int f = 0; f < SUM_MAXF; ++f) {
-    mx[f] = -1.0e16f; mn[f] = 1.0e16f; kx[f] = kn[f] = NONE; sm[f] = raw[f] = 0.0; nnan[f] = ninf[f] = 0;
+    mx[f] = -1.0e16f; mn[f] = 1.0e16f; kx[f] = kn[f] = SUM_NONE; sm[f] = raw[f] = 0.0; nnan[f] = ninf[f] = 0;
   }
-  const int n = Nx * Ny;
-  for (int c = threadIdx.x; c < n; c += SUM_NT) {
-    const int y = c / Nx, x = c - y * Nx;
+  for (long i = (long)blockIdx.y * chunk + threadIdx.x; i < i1; i += STAT_NT) {
+    const int y = (int)(i / g), x = 4 * (int)(i - (long)y * g);
     const long o = (long)z * ps + (long)y * P + x;
-    const long long key = ((long long)x * Ny + y) * Nz + z;
-    const float rho = S[o];
-    const float rinv = (float)(1.0 / (double)rho);
+    float rinv[4];
+    double dc[4] = {1.0, 1.0, 1.0, 1.0};
+    if (dcol) {                                 /* terrain: D per cell */
+      const float4 t = *(const float4 *)(dcol + (long)(z + 3) * ps + (long)y * P + x);
+      dc[0] = t.x; dc[1] = t.y; dc[2] = t.z; dc[3] = t.w;
+    }
 #pragma unroll
     for (int f = 0; f < SUM_MAXF; ++f) {
       if (f >= ns) break;
       /* rows: rho, u, v, w, theta, p', TKE..., moisture... */
-      float fr;
-      if (f < 5) fr = S[(long)f * fs + o];
-      else if (f == 5) fr = pres ? pres[o] : 0.f;
-      else fr = S[(long)(f - 1) * fs + o];
+      float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (f < 5) t = *(const float4 *)(S + (long)f * fs + o);
+      else if (f == 5) { if (pres) t = *(const float4 *)(pres + o); }
+      else t = *(const float4 *)(S + (long)(f - 1) * fs + o);
+      const float fr[4] = {t.x, t.y, t.z, t.w};
       const bool cons = (f != 0 && f != 5);
-      const float v = cons ? fr * rinv : fr;
-      if (dcol) raw[f] += (double)fr * (double)dcol[(long)(z + 3) * ps + (long)y * P + x];   /* terrain: D per cell */
-      else raw[f] += (double)fr;
-      if (isnan(v)) { nnan[f]++; continue; }
-      if (isinf(v)) { ninf[f]++; continue; }
-      sum_pick(mx[f], kx[f], v, key, true);
-      sum_pick(mn[f], kn[f], v, key, false);
-      sm[f] += (double)v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (f == 0) rinv[j] = (float)(1.0 / (double)fr[j]);
+        if (x + j >= Nx) continue;              /* the row's padding */
+        const float v = cons ? fr[j] * rinv[j] : fr[j];
+        raw[f] += dcol ? (double)fr[j] * dc[j] : (double)fr[j];
+        if (isnan(v)) { nnan[f]++; continue; }
+        if (isinf(v)) { ninf[f]++; continue; }
+        const unsigned key = (unsigned)(x + j) * (unsigned)Ny + (unsigned)y;
+        sum_pick(mx[f], kx[f], v, key, true);
+        sum_pick(mn[f], kn[f], v, key, false);
+        sm[f] += (double)v;
+      }
     }
   }
   /* wavefront reduction */
 #pragma unroll
   for (int f = 0; f < SUM_MAXF; ++f) {
+    if (f >= ns) break;
     for (int off = 32; off > 0; off >>= 1) {
       sum_pick(mx[f], kx[f], __shfl_xor(mx[f], off), __shfl_xor(kx[f], off), true);
       sum_pick(mn[f], kn[f], __shfl_xor(mn[f], off), __shfl_xor(kn[f], off), false);
@@ -1382,7 +1487,7 @@ __global__ void __launch_bounds__(SUM_NT) k_summary(const float *S, const float 
       ninf[f] += __shfl_xor(ninf[f], off);
     }
   }
-  __shared__ double part[SUM_NT / 64][SUM_MAXF][SUM_LV];
+  __shared__ double part[STAT_NT / 64][SUM_MAXF][SUM_LV];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   if (lane == 0) {
 #pragma unroll
@@ -1393,19 +1498,15 @@ __global__ void __launch_bounds__(SUM_NT) k_summary(const float *S, const float 
     }
   }
   __syncthreads();
-  if (threadIdx.x < ns) {
-    const int f = threadIdx.x;
-    float vx = (float)part[0][f][0], vn = (float)part[0][f][2];
-    long long qx = (long long)part[0][f][1], qn = (long long)part[0][f][3];
-    double a4 = part[0][f][4], a5 = part[0][f][5], a6 = part[0][f][6], a7 = part[0][f][7];
-    for (int wv = 1; wv < SUM_NT / 64; ++wv) {
-      sum_pick(vx, qx, (float)part[wv][f][0], (long long)part[wv][f][1], true);
-      sum_pick(vn, qn, (float)part[wv][f][2], (long long)part[wv][f][3], false);
-      a4 += part[wv][f][4]; a5 += part[wv][f][5]; a6 += part[wv][f][6]; a7 += part[wv][f][7];
-    }
-    double *r = out + ((long)z * ns + f) * SUM_LV;
-    r[0] = vx; r[1] = (double)qx; r[2] = vn; r[3] = (double)qn; r[4] = a4; r[5] = a5; r[6] = a6; r[7] = a7;
-  }
+  if (threadIdx.x < ns)
+    summary_join(&part[0][threadIdx.x][0], SUM_MAXF * SUM_LV, STAT_NT / 64,
+                 out + (((long)blockIdx.y * gridDim.x + z) * ns + threadIdx.x) * SUM_LV);
+}
+/* A level's parts joined into part 0's row, in place. */
+__global__ void __launch_bounds__(64) k_summary_final(double *out, int parts, int nlev, int ns) {
+  if (threadIdx.x >= ns) return;
+  double *r = out + ((long)blockIdx.x * ns + threadIdx.x) * SUM_LV;
+  summary_join(r, (long)nlev * ns * SUM_LV, parts, r);
 }
 
 int fe_state_summary(double *out, int nrow) {
@@ -1413,19 +1514,19 @@ int fe_state_summary(double *out, int nrow) {
   const int ns = 6 + D.nTKE + D.nM;
   if (nrow != ns || !out || ns > SUM_MAXF) return FE_ERR_UNSUPPORTED;
   std::vector<double> lv((size_t)D.Nz * ns * SUM_LV);
-  double *d = nullptr;
-  HIPCHK(hipMalloc(&d, lv.size() * sizeof(double)));
+  const long n4 = (long)((D.Nx + 3) / 4) * D.Ny;
+  const int parts = stat_parts(D.Nz, n4, LONG_MAX);
+  int rc;
+  if ((rc = stat_space((size_t)parts * lv.size()))) return rc;
   /* on a terrain-following grid the kernel weights each cell by its own D (row PR_D of the
    * per-column table); on a flat one the host multiplies the level sums by the level's D */
   const float *dcol = D.terrain ? D.tprof + (size_t)PR_D * D.np * D.ps : nullptr;
-  hipLaunchKernelGGL(k_summary, dim3(D.Nz), dim3(SUM_NT), 0, D.stream, D.S[0], D.pout, D.fs, D.ps, D.Nx, D.Ny, D.Nz, D.P, ns,
-                     D.nTKE, d, dcol);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(lv.data(), d, lv.size() * sizeof(double), hipMemcpyDeviceToHost, D.stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(D.stream);
-  const hipError_t ef = hipFree(d);
-  if (e == hipSuccess) e = ef;
-  HIPCHK(e);
+  hipLaunchKernelGGL(k_summary, dim3(D.Nz, parts), dim3(STAT_NT), 0, D.stream, D.S[0], D.pout, D.fs, D.ps, D.Nx, D.Ny, D.P, ns,
+                     (n4 + parts - 1) / parts, D.stat, dcol);
+  if (parts > 1) hipLaunchKernelGGL(k_summary_final, dim3(D.Nz), dim3(64), 0, D.stream, D.stat, parts, D.Nz, ns);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(lv.data(), D.stat, lv.size() * sizeof(double), hipMemcpyDeviceToHost, D.stream));
+  HIPCHK(hipStreamSynchronize(D.stream));
   const double NONE = (double)0x7fffffffffffffffLL;
   const double ncell = (double)D.Nx * D.Ny * D.Nz;
   const double dV = (double)dX * dY * dZ;
@@ -1436,7 +1537,10 @@ int fe_state_summary(double *out, int nrow) {
     for (int z = 0; z < D.Nz; ++z) {
       const double *r = &lv[((size_t)z * ns + f) * SUM_LV];
       const float v1 = (float)r[0], v2 = (float)r[2];
-      const long long k1 = (long long)r[1], k2 = (long long)r[3];
+      /* column x Ny + y of the level -> the reference's loop order over the grid */
+      const long long none = 0x7fffffffffffffffLL;
+      const long long k1 = r[1] >= (double)SUM_NONE ? none : (long long)r[1] * D.Nz + z;
+      const long long k2 = r[3] >= (double)SUM_NONE ? none : (long long)r[3] * D.Nz + z;
       if (v1 > vx || (v1 == vx && k1 < qx)) { vx = v1; qx = k1; }
       if (v2 < vn || (v2 == vn && k2 < qn)) { vn = v2; qn = k2; }
       sum += r[4]; nn += r[5]; ni += r[6];
