@@ -116,6 +116,12 @@ struct Dev {
   long probe_n = 0;
 } D;
 
+}  // namespace
+
+#include "fe_transfer.hip"
+
+namespace {
+
 /* A launch on the model's stream, timed as class cls while the event pool has room: the launch
  * carries its pair of events itself (hipExtLaunchKernelGGL takes them from the kernel's own
  * dispatch), where event records of their own between the launches would add about 7 us of wall
@@ -142,47 +148,66 @@ inline size_t padded_col(int x, int y) {
 
 /* --------------------------------------------------------------------------- */
 /* layout conversion kernels                                                    */
-__global__ void k_host_to_dev(const float *src, float *dst, int Nx, int Ny, int Nz, int Nh, int P, long ps) {
-  int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
-  if (x >= Nx) return;
+/* The host arrays are z fastest, the device planes x fastest: both conversions go through a 64 x 64
+ * tile of (x, z) at one y in LDS, so that either side is read and written in 256-byte runs
+ * (without it each lane touched a line of its own: 512 x 512 x 128, one field, 265 us up and
+ * 352 us down -> 76 and 99 us). */
+constexpr int TT = 64;
+__global__ void __launch_bounds__(256) k_host_to_dev(const float *src, float *dst, int Nx, int Ny, int Nz, int Nh, int P, long ps) {
+  __shared__ float t[TT][TT + 1];
   const long NYH = Ny + 2 * Nh, NZH = Nz + 2 * Nh;
-  dst[(long)z * ps + (long)y * P + x] = src[((long)(x + Nh) * NYH + (y + Nh)) * NZH + (z + Nh)];
+  const int l = threadIdx.x % TT, r = threadIdx.x / TT, x0 = blockIdx.x * TT, z0 = blockIdx.z * TT, y = blockIdx.y;
+  for (int i = r; i < TT; i += 256 / TT)
+    if (x0 + i < Nx && z0 + l < Nz) t[i][l] = src[((long)(x0 + i + Nh) * NYH + (y + Nh)) * NZH + (z0 + l + Nh)];
+  __syncthreads();
+  for (int i = r; i < TT; i += 256 / TT)
+    if (x0 + l < Nx && z0 + i < Nz) dst[(long)(z0 + i) * ps + (long)y * P + x0 + l] = t[l][i];
 }
 
 /* rule: 0 rho, 1 rho*u, 2 rho*v, 3 rho*w, 4 rho*theta, 5 sgs tke, 6 moisture (and other fields with
  * zero-gradient halos), 7 pressure, 8 interior only (zero halos) */
-__global__ void k_dev_to_host(const float *src, float *dst, int Nx, int Ny, int Nz, int Nh, int P, long ps, int rule,
-                              const float *prof, int np, float uTop, float vTop, const float *tprof, int NyS) {
-  const int NZH = Nz + 2 * Nh;
-  int k = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, i = blockIdx.z;
-  if (k >= NZH) return;
+__global__ void __launch_bounds__(256) k_dev_to_host(const float *src, float *dst, int Nx, int Ny, int Nz, int Nh, int P, long ps,
+                                                     int rule, const float *prof, int np, float uTop, float vTop,
+                                                     const float *tprof, int NyS) {
+  __shared__ float t[TT][TT + 1];
+  const int NXH = Nx + 2 * Nh, NZH = Nz + 2 * Nh;
   const long NYH = Ny + 2 * Nh;
-  int x = i - Nh, y = j - Nh, z = k - Nh;
+  const int l = threadIdx.x % TT, r = threadIdx.x / TT, i0 = blockIdx.x * TT, k0 = blockIdx.z * TT, j = blockIdx.y;
+  const int i = i0 + l;
+  int x = i - Nh, y = j - Nh;
   x = ((x % Nx) + Nx) % Nx;
   y = ((y % Ny) + Ny) % Ny;
   const long col = (long)y * P + x;
-  float v;
-  if (rule == 8 && (i < Nh || i >= Nx + Nh || j < Nh || j >= Ny + Nh || z < 0 || z >= Nz)) v = 0.f;
-  else if (z >= 0 && z < Nz) v = src[z * ps + col];
-  else if (tprof && (rule == 0 || rule == 4 || (z >= Nz && (rule == 1 || rule == 2)))) {
-    /* terrain-following grid: the column's own base state and top-halo momentum (with lateral
-     * halo storage, NyS > Ny, the table holds the lateral halo columns' own rows) */
-    const int row = rule == 0 ? PR_RHO : (rule == 4 ? PR_RTH : (rule == 1 ? PR_UTOP : PR_VTOP));
-    const int hx = i - Nh, hy = j - Nh;
-    const long tcol = (NyS > Ny && hx >= -3 && hx < Nx + 3 && hy >= -3 && hy < Ny + 3)
-                          ? (long)(hy < 0 ? hy + NyS : hy) * P + (hx < 0 ? hx + P : hx)
-                          : col;
-    v = tprof[((long)row * np + (z + 3)) * ps + tcol];
-  }
-  else if (rule == 0) v = prof[(z + 3) * PROW + PR_RHO];
-  else if (rule == 4) v = prof[(z + 3) * PROW + PR_RTH];
-  else if (rule == 7) v = (k == 0) ? 0.f : src[(z < 0 ? 0 : Nz - 1) * ps + col];
-  else if (z < 0) v = src[col];
-  else if (rule == 1) v = uTop;
-  else if (rule == 2) v = vTop;
-  else if (rule == 3 || rule == 5) v = 0.f;
-  else v = src[(long)(Nz - 1) * ps + col];
-  dst[((long)i * NYH + j) * NZH + k] = v;
+  auto value = [&](int k) -> float {
+    const int z = k - Nh;
+    float v;
+    if (rule == 8 && (i < Nh || i >= Nx + Nh || j < Nh || j >= Ny + Nh || z < 0 || z >= Nz)) v = 0.f;
+    else if (z >= 0 && z < Nz) v = src[z * ps + col];
+    else if (tprof && (rule == 0 || rule == 4 || (z >= Nz && (rule == 1 || rule == 2)))) {
+      /* terrain-following grid: the column's own base state and top-halo momentum (with lateral
+       * halo storage, NyS > Ny, the table holds the lateral halo columns' own rows) */
+      const int row = rule == 0 ? PR_RHO : (rule == 4 ? PR_RTH : (rule == 1 ? PR_UTOP : PR_VTOP));
+      const int hx = i - Nh, hy = j - Nh;
+      const long tcol = (NyS > Ny && hx >= -3 && hx < Nx + 3 && hy >= -3 && hy < Ny + 3)
+                            ? (long)(hy < 0 ? hy + NyS : hy) * P + (hx < 0 ? hx + P : hx)
+                            : col;
+      v = tprof[((long)row * np + (z + 3)) * ps + tcol];
+    }
+    else if (rule == 0) v = prof[(z + 3) * PROW + PR_RHO];
+    else if (rule == 4) v = prof[(z + 3) * PROW + PR_RTH];
+    else if (rule == 7) v = (k == 0) ? 0.f : src[(z < 0 ? 0 : Nz - 1) * ps + col];
+    else if (z < 0) v = src[col];
+    else if (rule == 1) v = uTop;
+    else if (rule == 2) v = vTop;
+    else if (rule == 3 || rule == 5) v = 0.f;
+    else v = src[(long)(Nz - 1) * ps + col];
+    return v;
+  };
+  for (int k = r; k < TT; k += 256 / TT)
+    if (i < NXH && k0 + k < NZH) t[k][l] = value(k0 + k);
+  __syncthreads();
+  for (int n = r; n < TT; n += 256 / TT)
+    if (i0 + n < NXH && k0 + l < NZH) dst[((long)(i0 + n) * NYH + j) * NZH + k0 + l] = t[l][n];
 }
 
 /* Lateral halo of a block with lateral halo storage (see cuda_gridInit) from the block's own
@@ -656,33 +681,29 @@ int one_step(float *pout_last) {
 }
 
 int upload_field(const float *host, float *dev) {
-  const long bytes = D.n3h * sizeof(float);
-  HIPCHK(hipMemcpyAsync(D.stg, host, bytes, hipMemcpyHostToDevice, D.stream));
-  dim3 g((D.Nx + 63) / 64, D.Ny, D.Nz);
-  hipLaunchKernelGGL(k_host_to_dev, g, dim3(64), 0, D.stream, D.stg, dev, D.Nx, D.Ny, D.Nz, D.Nh, D.P, D.ps);
+  int rc;
+  if ((rc = xfer_up(D.stream, D.stg, host, D.n3h * sizeof(float)))) return rc;
+  dim3 g((D.Nx + TT - 1) / TT, D.Ny, (D.Nz + TT - 1) / TT);
+  hipLaunchKernelGGL(k_host_to_dev, g, dim3(256), 0, D.stream, D.stg, dev, D.Nx, D.Ny, D.Nz, D.Nh, D.P, D.ps);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(D.stream));
   return FE_OK;
 }
 
 int download_field(const float *dev, float *host, int rule) {
-  const int NZH = D.Nz + 2 * D.Nh;
-  dim3 g((NZH + 63) / 64, D.Ny + 2 * D.Nh, D.Nx + 2 * D.Nh);
-  hipLaunchKernelGGL(k_dev_to_host, g, dim3(64), 0, D.stream, dev, D.stg, D.Nx, D.Ny, D.Nz, D.Nh, D.P, D.ps, rule, D.prof, D.np, D.uTop, D.vTop,
+  dim3 g((D.Nx + 2 * D.Nh + TT - 1) / TT, D.Ny + 2 * D.Nh, (D.Nz + 2 * D.Nh + TT - 1) / TT);
+  hipLaunchKernelGGL(k_dev_to_host, g, dim3(256), 0, D.stream, dev, D.stg, D.Nx, D.Ny, D.Nz, D.Nh, D.P, D.ps, rule, D.prof, D.np, D.uTop, D.vTop,
                      (const float *)(D.terrain ? D.tprof : nullptr), D.NyS);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(host, D.stg, D.n3h * sizeof(float), hipMemcpyDeviceToHost, D.stream));
-  HIPCHK(hipStreamSynchronize(D.stream));
-  return FE_OK;
+  return xfer_down(D.stream, host, D.stg, D.n3h * sizeof(float));
 }
 
 int upload_2d(const float *host, float *dev) {
   if (!host) return FE_OK;
-  HIPCHK(hipMemcpyAsync(D.stg, host, D.n2h * sizeof(float), hipMemcpyHostToDevice, D.stream));
+  int rc;
+  if ((rc = xfer_up(D.stream, D.stg, host, D.n2h * sizeof(float)))) return rc;
   dim3 g((D.Nx + 63) / 64, D.Ny);
   hipLaunchKernelGGL(k_2d_to_dev, g, dim3(64), 0, D.stream, D.stg, dev, D.Nx, D.Ny, D.Nh, D.P);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(D.stream));
   return FE_OK;
 }
 
@@ -691,9 +712,7 @@ int download_2d(const float *dev, float *host) {
   dim3 g((D.Ny + 2 * D.Nh + 63) / 64, D.Nx + 2 * D.Nh);
   hipLaunchKernelGGL(k_2d_to_host, g, dim3(64), 0, D.stream, dev, D.stg, D.Nx, D.Ny, D.Nh, D.P);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(host, D.stg, D.n2h * sizeof(float), hipMemcpyDeviceToHost, D.stream));
-  HIPCHK(hipStreamSynchronize(D.stream));
-  return FE_OK;
+  return xfer_down(D.stream, host, D.stg, D.n2h * sizeof(float));
 }
 
 float *field_ptr(float *S, int f) { return S + (long)f * D.fs; }
@@ -701,6 +720,8 @@ float *field_ptr(float *S, int f) { return S + (long)f * D.fs; }
 int upload_state(void) {
   int rc;
   const long n3 = D.n3h;
+  if ((rc = xfer_reserve(n3 * sizeof(float)))) return rc;
+  XferScope scope;
   for (int f = 0; f < 5; ++f)
     if ((rc = upload_field(hydroFlds + f * n3, field_ptr(D.S[0], f)))) return rc;
   for (int f = 0; f < D.nTKE; ++f)
@@ -718,12 +739,14 @@ int upload_state(void) {
       if ((rc = upload_2d(qFlux, surfp(SF_QF)))) return rc;
     }
   }
-  return FE_OK;
+  return xfer_finish(D.stream);
 }
 
 int download_state(int with_pres) {
   int rc;
   const long n3 = D.n3h;
+  if ((rc = xfer_reserve(n3 * sizeof(float)))) return rc;
+  XferScope scope;
   for (int f = 0; f < 5; ++f)
     if ((rc = download_field(field_ptr(D.S[0], f), hydroFlds + f * n3, f))) return rc;
   for (int f = 0; f < D.nTKE; ++f)
@@ -763,7 +786,7 @@ int download_state(int with_pres) {
       if ((rc = download_2d(surfp(SF_QSK), qskin))) return rc;
     }
   }
-  return FE_OK;
+  return xfer_finish(D.stream);
 }
 
 long idx3(int i, int j, int k) { return ((long)i * (Nyp + 2 * Nh) + j) * (Nzp + 2 * Nh) + k; }
@@ -795,6 +818,8 @@ int fecuda_Init(void) {
 }
 
 int fecuda_Cleanup(void) {
+  /* the pinned slots go with the model, unless an ensemble is being put together from models */
+  if (fe_ens_count() == 0) xfer_release();
   if (D.stream) { (void)hipStreamDestroy(D.stream); D.stream = nullptr; }
   D.fecuda = 0;
   return FE_OK;
@@ -1581,11 +1606,14 @@ int fe_debug_build_frhs(int stage) {
   for (int f = 0; f < D.nM; ++f) put(moistScalarsFrhs + f * n3, 5 + D.nTKE + f);
   /* surface-layer state was advanced by a physics stage; bring it back too */
   if (physics_stage(stage) && surflayerSelector > 0) {
+    if ((rc = xfer_reserve(D.n3h * sizeof(float)))) return rc;
+    XferScope scope;
     if ((rc = download_2d(surfp(SF_CD), cdFld))) return rc;
     if ((rc = download_2d(surfp(SF_CH), chFld))) return rc;
     if ((rc = download_2d(surfp(SF_UST), fricVel))) return rc;
     if ((rc = download_2d(surfp(SF_IOL), invOblen))) return rc;
     if ((rc = download_2d(surfp(SF_HF), htFlux))) return rc;
+    return xfer_finish(D.stream);
   }
   return FE_OK;
 }

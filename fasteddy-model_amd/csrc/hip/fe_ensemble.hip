@@ -244,6 +244,7 @@ int ens_free_all() {
   E.dirty = true;
   E.host_tab_newer = false;
   E.report.clear();
+  if (!D.fecuda) return xfer_release();        /* no model left to use the pinned slots */
   return FE_OK;
 }
 
@@ -355,9 +356,11 @@ int fe_ens_member_state(int m, float *out, long n) {
   if (m < 0 || m >= (int)E.mem.size() || !out) return FE_ERR_STATE;
   const Member &q = E.mem[m];
   if (n != (long)q.NF * q.fs) return FE_ERR_UNSUPPORTED;
-  HIPCHK(hipStreamSynchronize(E.stream));
-  HIPCHK(hipMemcpy(out, q.S[0], (size_t)n * sizeof(float), hipMemcpyDeviceToHost));
-  return FE_OK;
+  int rc;
+  if ((rc = xfer_reserve((size_t)n * sizeof(float)))) return rc;
+  XferScope scope;
+  if ((rc = xfer_down(E.stream, out, q.S[0], (size_t)n * sizeof(float)))) return rc;
+  return xfer_finish(E.stream);
 }
 
 /* Friction velocity plane of member m ([y][x], pitch P), n = Ny * P floats. */

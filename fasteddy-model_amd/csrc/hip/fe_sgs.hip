@@ -506,16 +506,30 @@ int fe_sgs_norm(float *buf, long n, int get) {
   return FE_OK;
 }
 
+/* n floats of a caller's rows to the device */
+static int sgs_rows_up(float *dev, const float *host, long n) {
+  const size_t bytes = n * sizeof(float);
+  int rc;
+  if (bytes < XF_LONE) {
+    HIPCHK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, sgs_stream()));
+    return FE_OK;
+  }
+  if ((rc = xfer_reserve(bytes))) return rc;
+  XferScope scope;
+  if ((rc = xfer_up(sgs_stream(), dev, host, bytes))) return rc;
+  return xfer_finish(sgs_stream());
+}
+
 /* Network forward of M normalised feature rows X ([M][256], host) into Y ([M][16], host). */
 int fe_mlp_forward(const float *X, long M, float *Y) {
   int rc;
   if (!X || !Y || M < 1) return FE_ERR_UNSUPPORTED;
   if (!G.have_w) return FE_ERR_STATE;
   if ((rc = sgs_rows(M))) return rc;
-  HIPCHK(hipMemcpy(G.Xb, X, M * SGS_KIN * sizeof(float), hipMemcpyHostToDevice));
+  if ((rc = sgs_rows_up(G.Xb, X, M * SGS_KIN))) return rc;
   if ((rc = mlp_forward(G.Xb, M))) return rc;
+  HIPCHK(hipMemcpyAsync(Y, G.Y, M * SGS_KOUT * sizeof(float), hipMemcpyDeviceToHost, sgs_stream()));
   HIPCHK(hipStreamSynchronize(sgs_stream()));
-  HIPCHK(hipMemcpy(Y, G.Y, M * SGS_KOUT * sizeof(float), hipMemcpyDeviceToHost));
   return FE_OK;
 }
 
@@ -528,19 +542,17 @@ int fe_mlp_gradient(const float *X, const float *T, long M, float *grad, double 
   if (!G.have_w) return FE_ERR_STATE;
   if ((rc = sgs_rows(M))) return rc;
   hipStream_t s = sgs_stream();
-  HIPCHK(hipMemcpy(G.Xb, X, M * SGS_KIN * sizeof(float), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(G.Tb, T, M * SGS_KOUT * sizeof(float), hipMemcpyHostToDevice));
+  if ((rc = sgs_rows_up(G.Xb, X, M * SGS_KIN))) return rc;
+  if ((rc = sgs_rows_up(G.Tb, T, M * SGS_KOUT))) return rc;
   HIPCHK(hipMemsetAsync(G.dloss, 0, sizeof(double), s));
   if ((rc = mlp_forward(G.Xb, M))) return rc;
   if ((rc = sgs_loss_grad(G.Tb, M))) return rc;
   if ((rc = mlp_backward(G.Xb, M))) return rc;
+  double l = 0.0;
+  HIPCHK(hipMemcpyAsync(grad, G.gw, NPARAM * sizeof(float), hipMemcpyDeviceToHost, s));
+  if (loss) HIPCHK(hipMemcpyAsync(&l, G.dloss, sizeof(double), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  HIPCHK(hipMemcpy(grad, G.gw, NPARAM * sizeof(float), hipMemcpyDeviceToHost));
-  if (loss) {
-    double l = 0.0;
-    HIPCHK(hipMemcpy(&l, G.dloss, sizeof(double), hipMemcpyDeviceToHost));
-    loss[0] = l / ((double)M * SGS_NOUT);
-  }
+  if (loss) loss[0] = l / ((double)M * SGS_NOUT);
   return FE_OK;
 }
 
