@@ -407,8 +407,7 @@ inline int physics_stage(int stage) { return (physics_oneRKonly == 0) || (stage 
 /* Split the column into z segments, one work-group per tile and segment, when the
  * tiles alone leave compute units idle: a stage work-group holds one compute unit
  * (its LDS), so fewer than 256 tiles (e.g. 256 x 256 cells = 128 tiles) would run
- * the chip at tiles/256.  Segments are even and at least 16 levels long (each costs
- * two warm-up levels); amd_zSegments > 0 sets the count. */
+ * the chip at tiles/256.  Segments are even; amd_zSegments > 0 sets the count. */
 /* Even segment length for n segments of Nz levels, and the segment count it gives. */
 static void seg_shape(int Nz, int n, int &len, int &nseg) {
   len = (Nz + n - 1) / n;
@@ -427,12 +426,11 @@ static int stage_wg_per_cu(const Variant &v) {
   return std::max(1, std::min(o1, o2));
 }
 
-/* A launch runs in rounds of (work-groups per CU) x CUs work-groups; a segment also computes
- * 2 warm-up levels below its first stored level and fills its pipeline (about 2 levels' worth
- * of set-up).  The count minimises rounds x (segment length + 4) over segments of at least 4
- * levels (fewest segments on ties): a count whose work-groups overflow the slots by a few
- * would add a nearly empty round, and a small grid gets enough work-groups to spread over the
- * CUs. */
+/* A launch runs in rounds of (work-groups per CU) x CUs work-groups; a segment also loads its
+ * window and fills its pipeline (about 2 levels' worth of set-up).  The count minimises rounds x
+ * (segment length + 2) over segments of at least 4 levels (fewest segments on ties): a count
+ * whose work-groups overflow the slots by a few would add a nearly empty round, and a small grid
+ * gets enough work-groups to spread over the CUs. */
 void choose_segments() {
   const int tiles = ((D.Nx + TX - 1) / TX) * ((D.Ny + TY - 1) / TY);
   static int ncu = 0;
@@ -452,7 +450,7 @@ void choose_segments() {
       seg_shape(D.Nz, c, len, nseg);
       if (c > 1 && len < 4) break;
       const long rounds = ((long)tiles * nseg + slots - 1) / slots;
-      const long cost = rounds * (len + (nseg > 1 ? 4 : 0));
+      const long cost = rounds * (len + (nseg > 1 ? 2 : 0));
       if (best < 0 || cost < best) { best = cost; n = c; }
     }
   }

@@ -263,6 +263,7 @@ struct Cfg {
   static constexpr int IQV = 5 + (TKE_ ? 1 : 0);
   static constexpr int IQL = IQV + 1;
   static constexpr int IQV_SAFE = NM_ > 0 ? IQV : 0;  /* in-range index for reads behind NM > 0 */
+  static constexpr int IE_SAFE = TKE_ ? IE : 0;
   static constexpr int SH = SH_, SE = SE_, SQV = SQV_, SQL = SQL_;
   static constexpr bool PHYS = PHYS_;
   static constexpr int NV = 4 + NM_;          /* u, v, w, theta, q/rho ... */
@@ -310,11 +311,13 @@ struct FaceLoop {
       FaceLoop<C, F + 1, FE>::yf(raw, gy, fy, fx, V, omb);
     }
   }
-  template <int WD>
+  /* z face below level z0 + J0 + 3, win[f][j] holding level z0 + j */
+  template <int WD, int J0>
   __device__ __forceinline__ static void zf(float (*win)[WD], float *gz, float W, const float *omb) {
     if constexpr (F < FE) {
-      gz[F] = face_flux<C::template sch<F>(), C::PHYS>(W, omb[F], win[F][1], win[F][2], win[F][3], win[F][4], win[F][5], win[F][6]);
-      FaceLoop<C, F + 1, FE>::template zf<WD>(win, gz, W, omb);
+      gz[F] = face_flux<C::template sch<F>(), C::PHYS>(W, omb[F], win[F][J0], win[F][J0 + 1], win[F][J0 + 2], win[F][J0 + 3],
+                                                       win[F][J0 + 4], win[F][J0 + 5]);
+      FaceLoop<C, F + 1, FE>::template zf<WD, J0>(win, gz, W, omb);
     }
   }
 };
@@ -574,14 +577,20 @@ __device__ __forceinline__ DynRows dyn_rows_up(const StepArgs &a, int z, unsigne
   return r;
 }
 
+/* Velocity through the z face between levels z and z + 1 (0 at the lid): D, J33, rho*w and rho^-1 of both. */
+__device__ __forceinline__ float zface_vel(const StepArgs &a, int z, float Dz, float J33z, float w, float rin, float Dp,
+                                           float J33p, float wp, float rinp) {
+  return (z + 1 >= a.Nz) ? 0.f : 0.5f * a.dZi * (Dp * J33p * wp * rinp + Dz * J33z * w * rin);
+}
+
 template <class C, int WD>
 __device__ __forceinline__ void dyn_tendency(const StepArgs &a, int z, const DynRows &R, float (*win)[WD], float rin, float rinp,
                                              float pzm, float pzp, float pgx, float pgy, const float *dxy,
                                              const float *gzlo, float *gzhi, const float *omb, float *F) {
   constexpr int NF = C::NF;
   const float Dz = R.Dz, Dp = R.Dp, J33z = R.J33z, J33p = R.J33p, invD = R.invD;
-  const float W = (z + 1 >= a.Nz) ? 0.f : 0.5f * a.dZi * (Dp * J33p * win[3][4] * rinp + Dz * J33z * win[3][3] * rin);
-  FaceLoop<C, 0>::template zf<WD>(win, gzhi, W, omb);
+  const float W = zface_vel(a, z, Dz, J33z, win[3][3], rin, Dp, J33p, win[3][4], rinp);
+  FaceLoop<C, 0>::template zf<WD, 1>(win, gzhi, W, omb);
 #pragma unroll
   for (int f = 0; f < NF; ++f) F[f] = -invD * (dxy[f] + (gzhi[f] - gzlo[f]));
   const float rho = win[0][3];
@@ -882,6 +891,28 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
     return cd * cd * sqrtf(fmaxf(0.f, t1 - fmaxf(0.f, N2 * 3.f)));
   };
 
+  /* SGS fluxes (tau_31, tau_32, tau_33, tau_theta3, moisture) through the own cell's (plane
+   * position X, Y) lower face of level lev, from its planes and those below: A = rho*Km, l, Delta, E = (2/3) rho*e and J33
+   * of level lev (cuda_sgsTurbDevice.cu:60-442) */
+  auto zflux = [&](int lev, int X, int Y, float A, float l, float delta, float E, float J33, float *zn) {
+    auto vp = [&](int q) -> Plane & { return VL(lev, q); };
+    auto vz = [&](int q) -> Plane & { return VL(lev - 1, q); };
+    const float Bv = A * fmaf(2.f * l, frcp(delta), 1.f);
+    float s33 = J33 * a.dZi * (vp(2)[Y][X] - vz(2)[Y][X]);
+    float s11 = a.dXi * (vp(0)[Y][X] - vp(0)[Y][X - 1]);
+    float s22 = a.dYi * (vp(1)[Y][X] - vp(1)[Y - 1][X]);
+    float s31 = 0.25f * (a.dXi * ((vp(2)[Y][X] - vp(2)[Y][X - 1]) + (vz(2)[Y][X] - vz(2)[Y][X - 1]))
+                       + J33 * a.dZi * ((vp(0)[Y][X] - vz(0)[Y][X]) + (vp(0)[Y][X - 1] - vz(0)[Y][X - 1])));
+    float s32 = 0.25f * (a.dYi * ((vp(2)[Y][X] - vp(2)[Y - 1][X]) + (vz(2)[Y][X] - vz(2)[Y - 1][X]))
+                       + J33 * a.dZi * ((vp(1)[Y][X] - vz(1)[Y][X]) + (vp(1)[Y - 1][X] - vz(1)[Y - 1][X])));
+    zn[0] = -2.f * A * s31;
+    zn[1] = -2.f * A * s32;
+    zn[2] = -2.f * A * s33 + (C::TKE ? (2.f / 3.f) * A * (s11 + s22 + s33) : 0.f) + E;
+    zn[3] = -Bv * J33 * a.dZi * (vp(3)[Y][X] - vz(3)[Y][X]);
+#pragma unroll
+    for (int m = 0; m < C::NM; ++m) zn[4 + m] = -Bv * J33 * a.dZi * (vp(4 + m)[Y][X] - vz(4 + m)[Y][X]);
+  };
+
   constexpr RingPlan PL = PLAN_PHYS;
   const Tile<C> T(a, tp, PL.r1);
   const int tid = T.tid, tx = T.tx, ty = T.ty, wave = T.wave, lane = T.lane;
@@ -893,11 +924,11 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
   auto lvl = [&](float (&v)[NF], int zz, unsigned cb) { T.lvl(a, v, zz, cb); };
   auto mfac = [&](float rho, float qv) { return T.mfac(a, rho, qv); };
 
-  /* The loop starts at level z0: 0 for the first z segment; two levels below the
-   * segment's first level zs otherwise, those levels being computed without output so
-   * that every value carried from level to level is in place when level zs is stored. */
-  const int zs = T.zs, ze = T.ze;
-  const int z0 = zs > 0 ? zs - 2 : 0;
+  /* The loop starts at the segment's first level z0.  What a level takes over from the one below
+   * (z fluxes through its lower face, rho*Km below, eddy viscosities) is formed by the set-up with
+   * the loop's own expressions, so a segment costs no level of its own (two levels run below the
+   * segment without output instead cost a 16-level segment 10%). */
+  const int z0 = T.zs, ze = T.ze;
 
   /* register window of the own column, z-3..z+3 */
   float win[NF][7];
@@ -931,6 +962,12 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
 #pragma unroll
   for (int f = 0; f < NF; ++f) gzlo[f] = 0.f;
   float rin = frcp(win[0][3]);
+  if (z0 > 0) {                                    /* z fluxes through the segment's lower face */
+    const float W = zface_vel(a, z0 - 1, cprof<C>(a, PR_D, z0 - 1, (unsigned)col), cprof<C>(a, PR_J33, z0 - 1, (unsigned)col),
+                              win[3][2], frcp(win[0][2]), cprof<C>(a, PR_D, z0, (unsigned)col),
+                              cprof<C>(a, PR_J33, z0, (unsigned)col), win[3][3], rin);
+    FaceLoop<C, 0>::template zf<7, 0>(win, gzlo, W, omb);
+  }
 
   /* ---- physics-stage carried state ---- */
   float zc[PH ? 4 + C::NM : 1];
@@ -955,6 +992,12 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
       sgs_lq<C>(a, z0 + 1, (unsigned)col, th[2], th[3], th[4], win[C::IE][4] * riz[3], l1, q1);
       kmo = a.c_k * 0.5f * (q0 + qm); lso = l0;
       kmo1 = a.c_k * 0.5f * (q1 + q0); lso1 = l1; qo1 = q1;
+      if (z0 > 0) {                                /* rho*Km of the level below the segment */
+        float l2, q2;
+        sgs_lq<C>(a, z0 - 2, (unsigned)col, win[4][0] * frcp(win[0][0]), th[0], th[1], win[C::IE][1] * riz[0], l2, q2);
+        const float km = a.c_k * 0.5f * (qm + q2);
+        Aown[0] = km * win[0][2];
+      }
       if (hasR1) {
         float t2[NF], t1[NF];
         lvl(t2, z0 - 2, hcolb);
@@ -979,22 +1022,22 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
         VL(z0 + lev, 1)[dy + 1][dx + 1] = t[2] * r;
         VL(z0 + lev, 2)[dy + 1][dx + 1] = t[3] * r;
         VL(z0 + lev, 3)[dy + 1][dx + 1] = t[4] * r;       /* level z0-1: the Smagorinsky N^2 */
-        if (lev == 0) {
 #pragma unroll
-          for (int m = 0; m < C::NM; ++m) VL(z0, 4 + m)[dy + 1][dx + 1] = t[C::IQV + m] * r;
-        }
+        for (int m = 0; m < C::NM; ++m) VL(z0 + lev, 4 + m)[dy + 1][dx + 1] = t[C::IQV + m] * r;
       }
     }
-    Aown[0] = 0.f;
     __syncthreads();
     if constexpr (!C::TKE) {                        /* Smagorinsky: K_m of level z0 from the planes */
       kmo = smag(z0, tx + 1, ty + 1, (unsigned)col);
       lso = cprof<C>(a, PR_DELTA, z0, (unsigned)col);
     }
     Aown[1] = kmo * win[0][3];
-    {
-      /* SGS fluxes through the lower face of level z0: the surface layer's at the ground
-       * (z0 = 0); for a later segment these only feed the first, unstored level */
+    if (z0 > 0) {
+      /* SGS fluxes through the lower face of a later segment: the loop's (zflux) */
+      zflux(z0, tx + 1, ty + 1, kmo * win[0][3], lso, cprof<C>(a, PR_DELTA, z0, (unsigned)col),
+            C::TKE ? (2.f / 3.f) * win[C::IE_SAFE][3] : 0.f, cprof<C>(a, PR_J33, z0, (unsigned)col), zc);
+    } else {
+      /* SGS fluxes through the ground: the surface layer's */
       auto v0 = [&](int q) -> Plane & { return VL(z0, q); };
       const int Y = ty + 1, X = tx + 1;
       float A = Aown[1];
@@ -1057,7 +1100,9 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
     if (hasR1) cDlH = cprof<C>(a, PR_DELTA, z0, (unsigned)T.hcol);
   }
   for (int z = z0; z < ze; ++z) {
-    const bool out = active && z >= zs;      /* levels below zs are the segment's warm-up */
+    /* always the same as active: a mask formed in each level leaves the compiler a better order
+     * of the level than the loop-invariant one (512 x 512 x 128 dry: 1080 -> 1060 us) */
+    const bool out = active && z >= T.zs;
     /* ---- loads (vector-memory waits are in order): the RK base of this level first, so
      *      that P3's wait for it leaves the prefetches in flight (two barrier phases cover
      *      its latency, and only one level of it is held in registers); then own level z+3
@@ -1333,25 +1378,9 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
           kmo1 = smag(z + 1, X, Y, (unsigned)col);
           lso1 = cprof<C>(a, PR_DELTA, z + 1, (unsigned)col);
         }
-        {
-          float A = kmo1 * win[0][4];
-          float Bv = A * fmaf(2.f * lso1, frcp(C::TERR ? tdelP : cprof<C>(a, PR_DELTA, z + 1, (unsigned)col)), 1.f);
-          float E = C::TKE ? (2.f / 3.f) * win[C::IE][4] : 0.f;
-          float s33 = J33p * a.dZi * (vp(2)[Y][X] - vz(2)[Y][X]);
-          float s11 = a.dXi * (vp(0)[Y][X] - vp(0)[Y][X - 1]);
-          float s22 = a.dYi * (vp(1)[Y][X] - vp(1)[Y - 1][X]);
-          float s31 = 0.25f * (a.dXi * ((vp(2)[Y][X] - vp(2)[Y][X - 1]) + (vz(2)[Y][X] - vz(2)[Y][X - 1]))
-                             + J33p * a.dZi * ((vp(0)[Y][X] - vz(0)[Y][X]) + (vp(0)[Y][X - 1] - vz(0)[Y][X - 1])));
-          float s32 = 0.25f * (a.dYi * ((vp(2)[Y][X] - vp(2)[Y - 1][X]) + (vz(2)[Y][X] - vz(2)[Y - 1][X]))
-                             + J33p * a.dZi * ((vp(1)[Y][X] - vz(1)[Y][X]) + (vp(1)[Y - 1][X] - vz(1)[Y - 1][X])));
-          zn[0] = -2.f * A * s31;
-          zn[1] = -2.f * A * s32;
-          zn[2] = -2.f * A * s33 + (C::TKE ? (2.f / 3.f) * A * (s11 + s22 + s33) : 0.f) + E;
-          zn[3] = -Bv * J33p * a.dZi * (vp(3)[Y][X] - vz(3)[Y][X]);
-#pragma unroll
-          for (int m = 0; m < C::NM; ++m) zn[4 + m] = -Bv * J33p * a.dZi * (vp(4 + m)[Y][X] - vz(4 + m)[Y][X]);
-          Aown[2] = A;
-        }
+        Aown[2] = kmo1 * win[0][4];
+        zflux(z + 1, X, Y, Aown[2], lso1, C::TERR ? tdelP : cprof<C>(a, PR_DELTA, z + 1, (unsigned)col),
+              C::TKE ? (2.f / 3.f) * win[C::IE_SAFE][4] : 0.f, J33p, zn);
         const float zdz = J33z * a.dZi;
         F[1] -= a.dXi * (tb1[0][ty][tx + 1] - tb1[0][ty][tx]) + a.dYi * (tb2[0][ty + 1][tx] - tb2[0][ty][tx]) + zdz * (zn[0] - zc[0]);
         F[2] -= a.dXi * (tb1[1][ty][tx + 1] - tb1[1][ty][tx]) + a.dYi * (tb2[1][ty + 1][tx] - tb2[1][ty][tx]) + zdz * (zn[1] - zc[1]);
@@ -1559,13 +1588,35 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
    *   pg[S]: horizontal p' differences of level it-2 (pg[S+1] written for it-1);
    *   gz: z flux through the lower face of level it-2;
    *   fx[S]: x flux through the own cell's low face at level it-2 (fx[S+1] written for it-1). */
-  /* A z segment [zs, ze) other than the first starts its pipeline at it0 = zs - 2: P1
-   * of levels zs-2 and zs-1 and P2/P3 of level zs-1 run without output, so that p',
-   * the plane buffers and the z flux through the segment's lower face are in place
-   * when level zs is stored. */
-  const int zs = T.zs, ze = T.ze;
-  const int it0 = zs > 0 ? zs - 2 : 0;
-  const int zlo = zs > 0 ? zs - 1 : 0;                /* lowest level whose P3 runs */
+  /* The pipeline starts at the segment's first level it0 and computes no plane or face outside
+   * [it0, ze): p' below the segment and the z flux through its lower face come from the set-up,
+   * formed with the loop's own expressions (64 x 64 x 48 in 12 segments of 4 levels: six
+   * iterations where two levels below the segment run without output made eight). */
+  const int it0 = T.zs, ze = T.ze;
+  float gz[NF], pp[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int f = 0; f < NF; ++f) gz[f] = 0.f;
+  /* from levels it0-3 .. it0+2: moist flat grids form it before the window is held (256 x 256 x 160:
+   * 331 us after it, 307 before), the others from the window (terrain-following 256 x 256 x 128:
+   * 227 us before, 215 from it; 64 x 64 x 48: 16.0 and 15.3) */
+  auto below = [&](float (&w6)[NF][6]) {
+    const float W = zface_vel(a, it0 - 1, cprof<C>(a, PR_D, it0 - 1, (unsigned)T.col), cprof<C>(a, PR_J33, it0 - 1, (unsigned)T.col),
+                              w6[3][2], frcp(w6[0][2]), cprof<C>(a, PR_D, it0, (unsigned)T.col),
+                              cprof<C>(a, PR_J33, it0, (unsigned)T.col), w6[3][3], frcp(w6[0][3]));
+    FaceLoop<C, 0>::template zf<6, 0>(w6, gz, W, T.omb);
+    pp[2] = pprime<C>(a, w6[4][2], T.mfac(a, w6[0][2], C::NM > 0 ? w6[C::IQV_SAFE][2] : 0.f), it0 - 1, (unsigned)T.col);
+  };
+  if (C::NM > 0 && !C::TERR && it0 > 0) {
+    float w6[NF][6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      float t[NF];
+      T.lvl(a, t, it0 + j - 3, colb);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) w6[f][j] = t[f];
+    }
+    below(w6);
+  }
   float win[NF][9];
   float hv[4][NF];
   /* the first segment's levels are compile-time constants (their boundary rules fold) */
@@ -1594,21 +1645,29 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
   };
   if (it0 == 0) init(0);
   else init(it0);
-  float bs[BSA ? 3 : 1][NF], gz[NF], fx[FXR ? 3 : 1][FXR ? NF : 1];
+  float bs[BSA ? 3 : 1][NF], fx[FXR ? 3 : 1][FXR ? NF : 1];
 #pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    gz[f] = 0.f;
+  for (int f = 0; f < NF; ++f)
     for (int l = 0; l < (BSA ? 3 : 1); ++l) bs[l][f] = 0.f;
-  }
   if constexpr (FXR)
 #pragma unroll
     for (int f = 0; f < NF; ++f) fx[0][f] = fx[1][f] = fx[2][f] = 0.f;
-  float pp[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
   float ri[4] = {0.f, 0.f, 0.f, 0.f};
   /* terrain-following grids: P1's base-state rows and D of level it (own column and ring-1
    * cell) in slot S, loaded one iteration ahead (slot S+1 for level it+1) */
   PRows pr1[C::TERR ? 3 : 1], prh[C::TERR ? 3 : 1];
   float d1[C::TERR ? 3 : 1], dh[C::TERR ? 3 : 1];
+  if (!(C::NM > 0 && !C::TERR) && it0 > 0) {
+    float w6[NF][6], t[NF];
+    T.lvl(a, t, it0 + 2, colb);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int j = 0; j < 5; ++j) w6[f][j] = win[f][j + 2];
+      w6[f][5] = t[f];
+    }
+    below(w6);
+  }
   if constexpr (C::TERR) {
     pr1[0] = p_rows<C>(a, it0, (unsigned)T.col);
     d1[0] = cprof<C>(a, PR_D, it0, (unsigned)T.col);
@@ -1651,12 +1710,12 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
     }
     /* ---- loads for the next level: RK base of level it-1, own level it+2, halo level it+2 ---- */
     if constexpr (BSA) {
-      if (z2 >= 0 && z2 < Nz && !a.emitF && !T.baseIn) {
+      if (z2 >= it0 && z2 < ze && !a.emitF && !T.baseIn) {
         const unsigned o2 = (unsigned)z2 * pb + colb;
 #pragma unroll
         for (int f = 0; f < NF; ++f) bs[S + 1][f] = T.ld_bs(f, o2);
       }
-    } else if (z3 >= zs && !a.emitF && !T.baseIn) {
+    } else if (z3 >= it0 && !a.emitF && !T.baseIn) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) bs[0][f] = T.ld_bs(f, o3);
     }
@@ -1666,21 +1725,25 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
 #pragma unroll
       for (int f = 0; f < NF; ++f) win[f][7 + S] = t[f];
     }
-    if (T.hasH && it + 2 < Nz) T.lvl(a, hv[S + 2], it + 2, hcolb);
+    if (T.hasH && it + 2 < ze) T.lvl(a, hv[S + 2], it + 2, hcolb);
 
-    /* ---- P1: plane, rho^-1 and p' of level it ---- */
+    /* ---- P1: plane, rho^-1 and p' of level it (above the segment rho^-1 and p' only) ---- */
     ri[S + 2] = frcp(win[0][5 + S]);
-    if (z1 < Nz) {
+    auto plane = [&]() {
 #pragma unroll
       for (int f = 0; f < NF; ++f) raw[b1][f][ty + HH][tx + HH] = win[f][5 + S];
       if (T.hasH) {
 #pragma unroll
         for (int f = 0; f < NF; ++f) (&raw[b1][f][0][0])[T.hslot] = hv[S][f];
       }
+    };
+    auto pown = [&]() {
       const float q = C::NM > 0 ? win[C::IQV_SAFE][5 + S] : 0.f;
       pp[S + 3] = C::TERR ? pprime_r<C>(a, win[4][5 + S], T.mfac(a, win[0][5 + S], q), pr1[S])
                           : pprime<C>(a, win[4][5 + S], T.mfac(a, win[0][5 + S], q), z1, (unsigned)T.col);
       if (it == 0) pp[S + 2] = pp[S + 3];            /* p'(-1) = p'(0) */
+    };
+    auto ring1 = [&]() {
       (&dvr[b1][0][0])[T.od] = C::TERR ? d1[S] * ri[S + 2] : ri[S + 2];
       (&dvp[b1][0][0])[T.od] = pp[S + 3];
       if (T.hasR1) {
@@ -1689,12 +1752,22 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
         (&dvp[b1][0][0])[T.hd] = C::TERR ? pprime_r<C>(a, hv[S][4], T.mfac(a, hv[S][0], qh), prh[S])
                                          : pprime<C>(a, hv[S][4], T.mfac(a, hv[S][0], qh), z1, (unsigned)T.hcol);
       }
-    } else {
-      pp[S + 3] = pp[S + 2];                         /* p'(Nz) = p'(Nz-1) */
+    };
+    if (z1 >= Nz) pp[S + 3] = pp[S + 2];             /* p'(Nz) = p'(Nz-1) */
+    if constexpr (C::NM > 0 || C::TERR) {
+      if (z1 < Nz) pown();
+      if (z1 < ze) {
+        plane();
+        ring1();
+      }
+    } else if (z1 < Nz) {                            /* one block: level ze's plane is written too and never read */
+      plane();
+      pown();
+      ring1();
     }
 
     /* ---- P2: x and y face fluxes of level it-1 ---- */
-    if (z2 >= 0 && z2 < Nz) {
+    if (z2 >= it0 && z2 < ze) {
       float (*rw)[RH][RW] = raw[b2];
       /* face velocities: the rho^-1 plane with the level's D factored out, or (terrain) the
        * plane of D rho^-1 */
@@ -1725,7 +1798,7 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
     }
 
     /* ---- P3: own cell of level it-2 ---- */
-    if (z3 >= zlo) {
+    if (z3 >= it0) {
       float dxy[NF], gzhi[NF], F[NF];
       float (*wv)[9] = win;
       float w7[NF][7];
@@ -1748,14 +1821,12 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
                          dxy, gz, gzhi, T.omb, F);
 #pragma unroll
       for (int f = 0; f < NF; ++f) gz[f] = gzhi[f];
-      if (z3 >= zs) {                                 /* uniform: not a warm-up level */
-        if (T.active) {
-          float b0[NF];
+      if (T.active) {
+        float b0[NF];
 #pragma unroll
-          for (int f = 0; f < NF; ++f) b0[f] = T.baseIn ? win[f][3 + S] : bs[BSA ? S : 0][f];
-          rk_store<C, EMIT>(a, T, o3, F, b0);
-          if (a.pout) *(float *)((char *)a.pout + o3) = pp[S + 1];
-        }
+        for (int f = 0; f < NF; ++f) b0[f] = T.baseIn ? win[f][3 + S] : bs[BSA ? S : 0][f];
+        rk_store<C, EMIT>(a, T, o3, F, b0);
+        if (a.pout) *(float *)((char *)a.pout + o3) = pp[S + 1];
       }
     }
     __syncthreads();
