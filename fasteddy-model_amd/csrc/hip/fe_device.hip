@@ -21,6 +21,8 @@
 #include <math.h>
 #include <algorithm>
 #include <array>
+#include <functional>
+#include <map>
 #include <random>
 #include <string>
 #include <stdio.h>

@@ -35,6 +35,7 @@ namespace {
 struct Member {
   int Nx = 0, Ny = 0, Nz = 0, P = 0, NF = 0, nseg = 1, zseg = 0, ntx = 0, nty = 0, mptf = 0;
   int nseg_plain = 1, zseg_plain = 0;   /* the plain path's own segments for this grid (timed baseline) */
+  bool seg_set = false;                 /* segments set by amd_zSegments, fe_ens_set_segments or the autotuner */
   long fs = 0, ps = 0;
   float *S[3] = {nullptr, nullptr, nullptr};
   float *prof = nullptr, *surf = nullptr;
@@ -54,6 +55,7 @@ struct Ens {
   unsigned *dctr = nullptr;
   EnsQueues Q;
   int nwg = 0;
+  bool seg_old = false;         /* members came since the default segments were chosen */
   bool dirty = true;            /* work items or kernel arguments changed: rebuild and recapture */
   bool host_tab_newer = false;  /* the host rows advanced (sequential steps): upload before a replay */
   hipGraph_t graph = nullptr;
@@ -75,6 +77,64 @@ void ens_set_segments(Member &m, int n) {
   seg_shape(m.Nz, n, m.zseg, m.nseg);
   for (int s = 0; s < 3; ++s) m.args[s].zseg = m.zseg;
   E.dirty = true;
+}
+
+/* Work-groups the chip holds at once: the persistent grid. */
+int ens_slots() {
+  int dev = 0, ncu = 256;
+  hipDeviceProp_t pr;
+  if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&pr, dev) == hipSuccess && pr.multiProcessorCount > 0)
+    ncu = pr.multiProcessorCount;
+  int o1 = 0, o2 = 0, occ = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o1, E.var.ens_phys, NT, 0) == hipSuccess &&
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&o2, E.var.ens_plain, NT, 0) == hipSuccess)
+    occ = std::max(1, std::min(o1, o2));
+  return ncu * occ;
+}
+
+/* Levels' worth of a work item: its levels and about two for loading its window and filling the
+ * pipeline. */
+inline int ens_item_cost(int levels) { return levels + 2; }
+
+/* Segments of the members that have none set: the segment length, of all even lengths >= 4, whose
+ * work items end earliest when the work-groups of the persistent grid take them longest first
+ * (longest length on ties).  A lone run's own choice spreads one member over the whole chip; here
+ * the members fill it together, and segments as short as a lone 64 x 64 x 48 member's (4 levels)
+ * spend a third of their items on set-up.  Measured in ms a step, lone-run choice -> this one: 16 of
+ * 64 x 64 x 48 0.399 (12 segments) -> 0.335 (2); 40 of them 0.928 -> 0.765 (4); eight of 96^2 x 64 to
+ * 192^2 x 96 within 1% of the best length of 8, 12, 16, 24, 32, 48, 64 levels, 48 of them within 3%. */
+void ens_default_segments() {
+  if (!E.seg_old) return;
+  E.seg_old = false;
+  const int slots = ens_slots();
+  int mz = 0;
+  for (auto &m : E.mem)
+    if (!m.seg_set) mz = std::max(mz, m.Nz);
+  long best = -1;
+  int blen = 0;
+  for (int len = 4; len < mz + 2; len += 2) {
+    std::map<int, long, std::greater<int>> items;      /* item cost -> items */
+    for (auto &m : E.mem) {
+      const long tiles = (long)((m.Nx + TX - 1) / TX) * ((m.Ny + TY - 1) / TY);
+      int zseg = m.zseg, nseg = m.nseg;
+      if (!m.seg_set) seg_shape(m.Nz, (m.Nz + len - 1) / len, zseg, nseg);
+      items[ens_item_cost(std::min(zseg, m.Nz))] += tiles * (nseg - 1);
+      items[ens_item_cost(m.Nz - (nseg - 1) * zseg)] += tiles;
+    }
+    std::map<long, long> load{{0, slots}};              /* work taken -> work-groups */
+    for (auto &it : items)
+      for (long left = it.second; left > 0;) {
+        const auto lo = load.begin();
+        const long at = lo->first, n = std::min(left, lo->second);
+        if ((lo->second -= n) == 0) load.erase(lo);
+        load[at + it.first] += n;
+        left -= n;
+      }
+    const long end = load.rbegin()->first;
+    if (best < 0 || end <= best) { best = end; blen = len; }
+  }
+  for (auto &m : E.mem)
+    if (!m.seg_set) ens_set_segments(m, (m.Nz + blen - 1) / blen);
 }
 
 int ens_drop_graph() {
@@ -105,6 +165,7 @@ int ens_build() {
   int rc;
   const int nm = (int)E.mem.size();
   if (nm == 0) return FE_ERR_STATE;
+  ens_default_segments();
   /* the tables below are freed and rewritten by null-stream calls, which do not wait for the
    * (non-blocking) ensemble stream */
   HIPCHK(hipStreamSynchronize(E.stream));
@@ -116,7 +177,7 @@ int ens_build() {
     m.nty = (m.Ny + TY - 1) / TY;
     for (int bz = 0; bz < m.nseg; ++bz) {
       const int z0 = bz * m.zseg, z1 = std::min(m.Nz, z0 + m.zseg);
-      const int cost = (z1 - z0) + (bz > 0 ? 2 : 0) + 2;   /* levels computed, pipeline set-up */
+      const int cost = ens_item_cost(z1 - z0);
       for (int b = 0; b < m.ntx * m.nty; ++b) t.push_back({EnsItem{i, b, m.ntx, bz}, cost});
     }
   }
@@ -159,18 +220,7 @@ int ens_build() {
   E.Q.tab = E.dtab;
   E.Q.items = E.ditems;
   E.Q.ctr = E.dctr;
-  /* persistent grid: as many work-groups as the compute units hold at once */
-  {
-    int dev = 0, ncu = 256, occ = 1;
-    hipDeviceProp_t pr;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&pr, dev) == hipSuccess && pr.multiProcessorCount > 0)
-      ncu = pr.multiProcessorCount;
-    int o1 = 0, o2 = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o1, E.var.ens_phys, NT, 0) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&o2, E.var.ens_plain, NT, 0) == hipSuccess)
-      occ = std::max(1, std::min(o1, o2));
-    E.nwg = ncu * occ;
-  }
+  E.nwg = ens_slots();
   if ((rc = ens_drop_graph())) return rc;
   HIPCHK(hipStreamBeginCapture(E.stream, hipStreamCaptureModeThreadLocal));
   rc = ens_enqueue_step();
@@ -316,6 +366,7 @@ int fe_ens_add_member(void) {
   m.Nx = D.Nx; m.Ny = D.Ny; m.Nz = D.Nz; m.P = D.P; m.NF = D.NF; m.fs = D.fs; m.ps = D.ps;
   m.nseg = D.nseg; m.zseg = D.zseg;
   m.nseg_plain = D.nseg; m.zseg_plain = D.zseg;
+  m.seg_set = amd_zSegments > 0;
   for (int s = 0; s < 3; ++s) m.S[s] = D.S[s];
   m.prof = D.prof;
   m.surf = D.surf;
@@ -336,6 +387,7 @@ int fe_ens_add_member(void) {
   D.grid = 0;
   E.mem.push_back(m);
   E.dirty = true;
+  E.seg_old = true;
   return (int)E.mem.size() - 1;
 }
 
@@ -345,6 +397,7 @@ int fe_ens_count(void) { return (int)E.mem.size(); }
  * step index, simulation time * 1000 (ms, rounded) */
 int fe_ens_member_info(int m, int *info, int n) {
   if (m < 0 || m >= (int)E.mem.size() || !info || n < 9) return FE_ERR_STATE;
+  ens_default_segments();
   const Member &q = E.mem[m];
   const int v[9] = {q.Nx, q.Ny, q.Nz, q.P, q.NF, q.nseg, q.zseg, q.args[0].step_it, (int)lroundf(q.args[0].simTime * 1000.f)};
   for (int i = 0; i < 9; ++i) info[i] = v[i];
@@ -377,6 +430,7 @@ int fe_ens_member_ustar(int m, float *out, long n) {
 int fe_ens_set_segments(int m, int nseg) {
   if (m < 0 || m >= (int)E.mem.size() || nseg < 1) return FE_ERR_STATE;
   ens_set_segments(E.mem[m], nseg);
+  E.mem[m].seg_set = true;
   return FE_OK;
 }
 
@@ -433,7 +487,7 @@ int fe_ens_step_times(int nsteps, int sequential, float *ms) {
 
 /* Autotuner: for each member shape (Nx, Ny, Nz) in turn, time trial_steps graph replays
  * for every z-segment count whose segments are at least 4 levels long and keep the
- * fastest (coordinate descent from the plain path's choice, two passes).  The members'
+ * fastest (coordinate descent from the segments the members have, two passes).  The members'
  * state, surface planes and step rows are saved first and restored after, so tuning
  * leaves the simulation where it was.  A report of the trials and choices is copied
  * into report (len bytes). */
@@ -461,7 +515,10 @@ int fe_ens_autotune(int trial_steps, char *report, int len) {
   }
   auto set_shape = [&](const std::array<int, 3> &s, int n) {
     for (auto &m : E.mem)
-      if (m.Nx == s[0] && m.Ny == s[1] && m.Nz == s[2]) ens_set_segments(m, n);
+      if (m.Nx == s[0] && m.Ny == s[1] && m.Nz == s[2]) {
+        ens_set_segments(m, n);
+        m.seg_set = true;
+      }
   };
   auto cur = [&](const std::array<int, 3> &s) {
     for (auto &m : E.mem)
