@@ -50,9 +50,39 @@ struct GemmArgs {
 
 constexpr int GT = 64, GK = 32, GKP = GK + 4;
 
-/* GELU and its derivative (below) */
-__device__ __forceinline__ float gelu(float z);
-__device__ __forceinline__ float gelu_d(float z);
+/* GELU(z) = z Phi(z) without transcendentals: Phi(z) = 1/2 + zc Q(zc^2), zc = z clamped to
+ * [-4, 4], Q a degree-7 polynomial (in zc^2) fitted to the normal CDF on [0, 4] in the
+ * weighted least-squares sense with Q(16) = 1/8 imposed, so that Phi = 0 and 1 beyond the
+ * clamp (to 5e-9): |GELU - z Phi_exact(z)| <= 1.4e-4 for all z (largest at |z| = 4, where the exact
+ * tail 4 Phi(-4) = 1.3e-4 is dropped), below half a BF16 step of any activation above 0.035,
+ * and 11 instructions against two quarter-rate transcendentals and 16 instructions of an
+ * erf-based form.  Q(s) = sum_j c_j s^j; c_0 = 0.39881 ~ 1/sqrt(2 pi). */
+__device__ __forceinline__ float gelu_q(float s) {
+  float q = fmaf(-1.288297990e-09f, s, 1.050534689e-07f);
+  q = fmaf(q, s, -3.724001524e-06f);
+  q = fmaf(q, s, 7.636147270e-05f);
+  q = fmaf(q, s, -1.022127353e-03f);
+  q = fmaf(q, s, 9.584851178e-03f);
+  q = fmaf(q, s, -6.606890165e-02f);
+  return fmaf(q, s, 3.988074278e-01f);
+}
+__device__ __forceinline__ float gelu(float z) {
+  const float zc = fminf(fmaxf(z, -4.f), 4.f);
+  return z * fmaf(zc, gelu_q(zc * zc), 0.5f);
+}
+/* its derivative Phi(z) + z Phi'(z): Phi' = d/dz [zc Q(zc^2)] = sum_j (2j+1) c_j zc^2j inside
+ * the clamp and 0 outside, so that the training gradient is that of the function evaluated */
+__device__ __forceinline__ float gelu_d(float z) {
+  const float zc = fminf(fmaxf(z, -4.f), 4.f), s = zc * zc;
+  float d = fmaf(-1.932446985e-08f, s, 1.365695096e-06f);
+  d = fmaf(d, s, -4.096401676e-05f);
+  d = fmaf(d, s, 6.872532543e-04f);
+  d = fmaf(d, s, -7.154891471e-03f);
+  d = fmaf(d, s, 4.792425589e-02f);
+  d = fmaf(d, s, -1.982067049e-01f);
+  d = fmaf(d, s, 3.988074278e-01f);
+  return fmaf(zc, gelu_q(s), 0.5f) + (fabsf(z) < 4.f ? z * d : 0.f);
+}
 
 /* Four consecutive values of an operand tile: element (r, c) at p + r*ld + c, c the unit-stride
  * index; columns at or past nc and rows at or past nr are 0.  vec: 16-byte loads are aligned. */
@@ -183,40 +213,6 @@ __global__ void __launch_bounds__(256) k_gemm_reduce(const float *part, int nz, 
 #pragma unroll 8
   for (int z = 0; z < nz; ++z) s += part[(long)z * n + i];
   out[i] = s;
-}
-
-/* GELU(z) = z Phi(z) without transcendentals: Phi(z) = 1/2 + zc Q(zc^2), zc = z clamped to
- * [-4, 4], Q a degree-7 polynomial (in zc^2) fitted to the normal CDF on [0, 4] in the
- * weighted least-squares sense with Q(16) = 1/8 imposed, so that Phi = 0 and 1 beyond the
- * clamp (to 5e-9): |GELU - z Phi_exact(z)| <= 1.4e-4 for all z (largest at |z| = 4, where the exact
- * tail 4 Phi(-4) = 1.3e-4 is dropped), below half a BF16 step of any activation above 0.035,
- * and 11 instructions against two quarter-rate transcendentals and 16 instructions of an
- * erf-based form.  Q(s) = sum_j c_j s^j; c_0 = 0.39881 ~ 1/sqrt(2 pi). */
-__device__ __forceinline__ float gelu_q(float s) {
-  float q = fmaf(-1.288297990e-09f, s, 1.050534689e-07f);
-  q = fmaf(q, s, -3.724001524e-06f);
-  q = fmaf(q, s, 7.636147270e-05f);
-  q = fmaf(q, s, -1.022127353e-03f);
-  q = fmaf(q, s, 9.584851178e-03f);
-  q = fmaf(q, s, -6.606890165e-02f);
-  return fmaf(q, s, 3.988074278e-01f);
-}
-__device__ __forceinline__ float gelu(float z) {
-  const float zc = fminf(fmaxf(z, -4.f), 4.f);
-  return z * fmaf(zc, gelu_q(zc * zc), 0.5f);
-}
-/* its derivative Phi(z) + z Phi'(z): Phi' = d/dz [zc Q(zc^2)] = sum_j (2j+1) c_j zc^2j inside
- * the clamp and 0 outside, so that the training gradient is that of the function evaluated */
-__device__ __forceinline__ float gelu_d(float z) {
-  const float zc = fminf(fmaxf(z, -4.f), 4.f), s = zc * zc;
-  float d = fmaf(-1.932446985e-08f, s, 1.365695096e-06f);
-  d = fmaf(d, s, -4.096401676e-05f);
-  d = fmaf(d, s, 6.872532543e-04f);
-  d = fmaf(d, s, -7.154891471e-03f);
-  d = fmaf(d, s, 4.792425589e-02f);
-  d = fmaf(d, s, -1.982067049e-01f);
-  d = fmaf(d, s, 3.988074278e-01f);
-  return fmaf(zc, gelu_q(s), 0.5f) + (fabsf(z) < 4.f ? z * d : 0.f);
 }
 
 /* mean-squared-error gradient over the first nout of N columns: dY = 2 (Y - T) / (M nout);
