@@ -428,19 +428,10 @@ __global__ void k_normalise(float *X, long M, int N, int nu, const float *mu, co
  * (every |normalised feature| <= gate) and the predicted stress tensor is realizable
  * (positive semi-definite: non-negative diagonal, |tau_ij|^2 <= tau_ii tau_jj, det >= 0,
  * Schumann 1977); its mask is 1 then, else 0. */
-__device__ __forceinline__ bool sgs_finish_cell(const float *y, const float *ymu, const float *ysd, float gm, float gate,
-                                                float rho, long c, float *tauL, long ncell, unsigned char *mask) {
-  float t[9];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) t[q] = y[q] * ysd[q] + ymu[q];
-  bool ok = gm <= gate;
-  const float a = t[0], b = t[1], d = t[2], e = t[3], f = t[4], h = t[5];
-  ok = ok && a >= 0.f && b >= 0.f && d >= 0.f && e * e <= a * b && f * f <= a * d && h * h <= b * d;
+__device__ __forceinline__ bool sgs_realizable(float a, float b, float d, float e, float f, float h) {
+  bool ok = a >= 0.f && b >= 0.f && d >= 0.f && e * e <= a * b && f * f <= a * d && h * h <= b * d;
   const float det = a * (b * d - h * h) - e * (e * d - h * f) + f * (e * h - b * f);
   ok = ok && det >= 0.f;
-  mask[c] = ok ? 1 : 0;
-#pragma unroll
-  for (int q = 0; q < 9; ++q) tauL[q * ncell + c] = rho * t[q];
   return ok;
 }
 
@@ -453,28 +444,43 @@ __global__ void k_sgs_finish(const float *Y, const float *ymu, const float *ysd,
   int x, y, z;
   cell_xyz(c, Nx, Ny, x, y, z);
   const float rho = S[(long)z * ps + (long)y * P + x];
-  sgs_finish_cell(Y + r * SGS_KOUT, ymu, ysd, gmax[c], gate, rho, c, tauL, ncell, mask);
+  float t[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) t[q] = Y[r * SGS_KOUT + q] * ysd[q] + ymu[q];
+  mask[c] = gmax[c] <= gate && sgs_realizable(t[0], t[1], t[2], t[3], t[4], t[5]) ? 1 : 0;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) tauL[q * ncell + c] = rho * t[q];
 }
 
 /* ---- fused inference ----------------------------------------------------------------------
  * Features, the four network layers and the finish of 64 cells per work-group iteration,
  * without the intermediate feature and activation arrays in HBM.  Persistent work-groups of
- * four waves: wave w keeps its 16 output columns of W1, W2, W3 (BF16, MFMA B-operand layout)
- * and all of W4 in registers for the whole launch and loops over tiles of 64 consecutive
- * cells (x-fastest interior index):
- *   features  thread (cell r = tid / 4, part p = tid % 4) reads the precomputed gradients
- *             of neighbours p, p+4, ... of the cell's 27 (and, p = 3, the seven dtheta/dz),
- *             normalises them, keeps their largest magnitude (the gate) and writes them as
- *             BF16 rows of the A tile in LDS;
- *   layers    4 row blocks x 16 (layer 1) or 4 (layers 2, 3) k blocks of
- *             v_mfma_f32_16x16x16_bf16 per wave, bias and GELU in FP32 on the accumulators,
- *             the activations back to LDS as BF16 for the next layer; layer 4: wave w the
- *             row block w, all 16 outputs;
- *   finish    one thread per cell: de-normalisation, gate, realizability, rho tau.
+ * four waves: wave w keeps its 16 output columns of W1, W2, W3 and all of W4 in registers (BF16)
+ * for the whole launch and loops over tiles of 64 consecutive cells (x-fastest interior index):
+ *   features  wave w, lane = cell: features 64 w .. 64 w + 63 from the precomputed gradients of
+ *             the eight neighbours that hold them (loaded one tile ahead, while the previous
+ *             tile is in layer 1), normalised, their largest magnitude (the
+ *             gate), four at a time as BF16 to LDS;
+ *   layers    4 cell blocks x 16 (layer 1) or 4 (layers 2, 3) k blocks of
+ *             v_mfma_f32_16x16x16_bf16 per wave with the weights as the left operand, so that a
+ *             lane holds four consecutive outputs of one cell: bias and GELU in FP32 on the
+ *             accumulators, then one 8-byte store of four BF16 activations for the next layer;
+ *             layer 4: wave w the cell block w, all 16 outputs;
+ *   finish    on the layer-4 accumulators: a lane de-normalises and stores its own outputs, the
+ *             first 16 lanes take the two off-diagonal stresses they lack from the next 16 and
+ *             decide gate and realizability.
+ * LDS holds operands as [k / 4][cell][4], so that both the stores and the operand reads are
+ * 8 bytes a lane over consecutive addresses.  Four barriers a tile: the next tile's features are
+ * written behind the one that ends layer 1.
  * The rounding points (features and activations to BF16, MFMA accumulation over k blocks in
  * increasing order, FP32 bias and GELU) are those of the unfused kernels, so both paths give
- * the same bits. */
-constexpr int FT = 64, AKP = SGS_KIN + 8, HKP = SGS_H + 8;
+ * the same bits.
+ * What bounds it: vector instructions, 970 per wave and tile (600 of them the GELUs), at two waves
+ * per SIMD (the prefetched features and the weights are 128 registers).
+ * 128 x 128 x 48: 234 us with four lanes per cell that read each feature's normalisation from LDS,
+ * stored it as two bytes and waited for every neighbour's loads, and a serial finish by one wave;
+ * 169 us so.  A contiguous run of tiles per XCD made no difference (170 us). */
+constexpr int FT = 64;
 
 struct FusedArgs {
   const float *G;                        /* [cells][12] from k_sgs_grad */
@@ -493,19 +499,110 @@ struct FusedArgs {
   int ntiles;
 };
 
-/* four consecutive BF16 values of an LDS row (8-byte aligned: row pitches and k offsets are
- * multiples of four elements) */
-__device__ __forceinline__ bf16x4 ld_frag(const unsigned short *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+typedef __bf16 bf16v2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned f2bf2(float a, float b) {
+  return __builtin_bit_cast(unsigned, bf16v2{(__bf16)a, (__bf16)b});
+}
+__device__ __forceinline__ bf16x4 ld_frag(const uint2 *p) { return __builtin_bit_cast(bf16x4, *p); }
 
-__global__ void __launch_bounds__(256) k_sgs_mlp_fused(FusedArgs a) {
-  __shared__ unsigned short As[FT][AKP];
-  __shared__ unsigned short Hs[2][FT][HKP];
-  __shared__ float Ys[FT][SGS_KOUT + 1];
-  __shared__ float gms[FT];
-  __shared__ float smu[SGS_KIN], sisd[SGS_KIN];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+/* The cell of a lane of the fused kernel: index and coordinates.  A work-group's tiles are a fixed
+ * number of cells apart, added with carries instead of two divisions a tile.  Cells past the end
+ * repeat the last one; nothing of theirs is stored. */
+struct TileCell {
+  long c;
+  int x, y, z;
+  __device__ __forceinline__ TileCell(const FusedArgs &a, long c0) {
+    c = min(c0, a.ncell - 1);
+    cell_xyz(c, a.Nx, a.Ny, x, y, z);
+  }
+  __device__ __forceinline__ void advance(const FusedArgs &a, long step, int sx, int sy, int sz) {
+    c += step;
+    x += sx;
+    y += sy;
+    z += sz;
+    if (x >= a.Nx) { x -= a.Nx; ++y; }
+    if (y >= a.Ny) { y -= a.Ny; ++z; }
+    if (c >= a.ncell) { c = a.ncell - 1; x = a.Nx - 1; y = a.Ny - 1; z = a.Nz - 1; }
+  }
+};
+
+/* One wave's share of a tile's features, W the wave: features 64 W .. 64 W + 63, lane = cell.
+ * Waves 0 to 2 need components of eight neighbours from their first on, wave 3 the last six
+ * neighbours and the seven dtheta/dz. */
+template <int W>
+struct TileFeatures {
+  static constexpr int N0 = SGS_H * W / 9, NN = W < 3 ? 8 : 6, TH = 9 * NN;
+  static_assert(SGS_H == FT && SGS_KIN == 4 * FT, "64 features per wave");
+  static_assert(W == 3 || 9 * (N0 + NN) >= 64 * (W + 1), "the neighbours hold the wave's features");
+  __device__ __forceinline__ static void load(const FusedArgs &a, const TileCell &p, float (&u)[72], float &rho) {
+    if (W == 0) rho = a.S[(long)p.z * a.ps + (long)p.y * a.P + p.x];
+    /* a neighbour's place is the cell's plus one step per direction, wrapped or clamped by the step
+     * (32 bits, modulo 2^32: the sum is a place in the grid) */
+    const unsigned c12 = 12u * (unsigned)p.c, row = 12u * (unsigned)a.Nx, plane = row * (unsigned)a.Ny;
+    const unsigned xo[3] = {p.x == 0 ? row - 12u : -12u, 0u, p.x == a.Nx - 1 ? 12u - row : 12u};
+    const unsigned yo[3] = {p.y == 0 ? plane - row : -row, 0u, p.y == a.Ny - 1 ? row - plane : row};
+    const unsigned zo[3] = {p.z == 0 ? 0u : -plane, 0u, p.z == a.Nz - 1 ? 0u : plane};
+    auto cell = [&](int dx, int dy, int dz) -> const float * { return a.G + (c12 + zo[dz + 1] + yo[dy + 1] + xo[dx + 1]); };
+#pragma unroll
+    for (int i = 0; i < NN; ++i) {
+      const int n = N0 + i;
+      const float4 *g4 = (const float4 *)cell(n % 3 - 1, (n / 3) % 3 - 1, n / 9 - 1);
+      const float4 u0 = g4[0], u1 = g4[1];
+      u[9 * i + 0] = u0.x; u[9 * i + 1] = u0.y; u[9 * i + 2] = u0.z; u[9 * i + 3] = u0.w;
+      u[9 * i + 4] = u1.x; u[9 * i + 5] = u1.y; u[9 * i + 6] = u1.z; u[9 * i + 7] = u1.w;
+      u[9 * i + 8] = ((const float *)g4)[8];
+    }
+    if constexpr (W == 3) {
+      /* dtheta/dz of the cell, x-, x+, y-, y+, z-, z+ (c_sgs_tnb) */
+      u[TH + 0] = cell(0, 0, 0)[9];
+      u[TH + 1] = cell(-1, 0, 0)[9];
+      u[TH + 2] = cell(1, 0, 0)[9];
+      u[TH + 3] = cell(0, -1, 0)[9];
+      u[TH + 4] = cell(0, 1, 0)[9];
+      u[TH + 5] = cell(0, 0, -1)[9];
+      u[TH + 6] = cell(0, 0, 1)[9];
+      /* the same last element in every wave's branch: the array stays in registers */
+#pragma unroll
+      for (int i = TH + 7; i < 72; ++i) u[i] = 0.f;
+    }
+  }
+  /* normalised, to As; returns their largest magnitude */
+  __device__ __forceinline__ static float put(const float2 *nrm, const float (&u)[72], uint2 (*As)[FT], int lane) {
+    float gm = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (i > 0 && i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+      float v[4];
+      const float4 n01 = *(const float4 *)&nrm[64 * W + 4 * i], n23 = *(const float4 *)&nrm[64 * W + 4 * i + 2];
+      const float mu[4] = {n01.x, n01.z, n23.x, n23.z}, isd[4] = {n01.y, n01.w, n23.y, n23.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int q = 64 * W + 4 * i + j;
+        if (q < SGS_NIN) {
+          const int k = q < 243 ? q - 9 * N0 : TH + q - 243;
+          v[j] = (u[k < 72 ? k : 0] - mu[j]) * isd[j];
+          gm = fmaxf(gm, fabsf(v[j]));
+        } else {
+          v[j] = 0.f;
+        }
+      }
+      As[16 * W + i][lane] = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+    }
+    return gm;
+  }
+};
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_sgs_mlp_fused(FusedArgs a) {
+  __shared__ uint2 As[SGS_KIN / 4][FT];        /* features     [k / 4][cell][4] */
+  __shared__ uint2 Hs[2][SGS_H / 4][FT];       /* activations, likewise */
+  __shared__ float gms[2][4][FT], rhos[2][FT]; /* by tile parity: each wave's largest feature, rho */
+  __shared__ __align__(16) float cf[4][SGS_H]; /* biases of layers 1-3; of layer 4, output std, output mean */
+  __shared__ __align__(16) float2 nrm[SGS_KIN];  /* feature normalisation: mean, 1 / std */
+  __shared__ unsigned cnts[4][2];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
-  /* B operands: lane holds B[k = 16 kb + 4 lk + v][n = lr] of its wave's column block */
+  /* weights as the left operand (its row = output column): lane holds W[k = 16 kb + 4 lk + v][n],
+   * n = lr of its wave's block (W4: n = lr) */
   bf16x4 w1[16], w2[4], w3[4], w4[4];
   const int ncol = 16 * wave + lr;
 #pragma unroll
@@ -524,131 +621,122 @@ __global__ void __launch_bounds__(256) k_sgs_mlp_fused(FusedArgs a) {
     w4[kb] = bf16x4{(short)f2bf(a.w[OW4_ + (k + 0) * SGS_KOUT + lr]), (short)f2bf(a.w[OW4_ + (k + 1) * SGS_KOUT + lr]),
                     (short)f2bf(a.w[OW4_ + (k + 2) * SGS_KOUT + lr]), (short)f2bf(a.w[OW4_ + (k + 3) * SGS_KOUT + lr])};
   }
-  const float b1 = a.w[OB1_ + ncol], b2 = a.w[OB2_ + ncol], b3 = a.w[OB3_ + ncol], b4 = a.w[OB4_ + lr];
-  for (int i = tid; i < SGS_KIN; i += 256) {
-    smu[i] = a.mu[i];
-    sisd[i] = a.isd[i];
+  for (int i = tid; i < SGS_KIN; i += 256) nrm[i] = make_float2(a.mu[i], a.isd[i]);
+  for (int i = tid; i < SGS_H; i += 256) {
+    cf[0][i] = a.w[OB1_ + i];
+    cf[1][i] = a.w[OB2_ + i];
+    cf[2][i] = a.w[OB3_ + i];
+    cf[3][i] = i < SGS_KOUT ? a.w[OB4_ + i] : i < 2 * SGS_KOUT ? a.ysd[i - SGS_KOUT] : i < 3 * SGS_KOUT ? a.ymu[i - 2 * SGS_KOUT] : 0.f;
   }
-  __syncthreads();
-  unsigned ncnt = 0, npass = 0;          /* cells finished and passing, by threads 0..63 */
-  for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
-    const long c0 = (long)tile * FT;
-    /* ---- features ---- */
-    {
-      const int r = tid >> 2, p = tid & 3;
-      const long c = c0 + r;
-      unsigned short *row = As[r];
-      float gm = 0.f;
-      if (c < a.ncell) {
-        int x, y, z;
-        cell_xyz(c, a.Nx, a.Ny, x, y, z);
-        auto cell = [&](int dx, int dy, int dz) -> const float * {
-          int xx = x + dx, yy = y + dy, zz = z + dz;
-          xx = xx < 0 ? xx + a.Nx : (xx >= a.Nx ? xx - a.Nx : xx);
-          yy = yy < 0 ? yy + a.Ny : (yy >= a.Ny ? yy - a.Ny : yy);
-          zz = zz < 0 ? 0 : (zz >= a.Nz ? a.Nz - 1 : zz);
-          return a.G + ((unsigned)(zz * a.Ny + yy) * (unsigned)a.Nx + (unsigned)xx) * 12u;
-        };
-        for (int n = p; n < 27; n += 4) {
-          const float4 *g4 = (const float4 *)cell(n % 3 - 1, (n / 3) % 3 - 1, n / 9 - 1);
-          const float4 u0 = g4[0], u1 = g4[1], u2 = g4[2];
-          const float g[9] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w, u2.x};
+  float u[72], rho = 0.f;                /* the wave's raw features of a tile (TileFeatures), rho (wave 0) */
 #pragma unroll
-          for (int k = 0; k < 9; ++k) {
-            const int q = 9 * n + k;
-            const float v = (g[k] - smu[q]) * sisd[q];
-            gm = fmaxf(gm, fabsf(v));
-            row[q] = f2bf(v);
-          }
-        }
-        if (p == 3) {
+  for (int i = 0; i < 72; ++i) u[i] = 0.f;
+  TileCell p(a, (long)blockIdx.x * FT + lane);
+  const long step = (long)gridDim.x * FT;
+  int sx, sy, sz;
+  cell_xyz(step, a.Nx, a.Ny, sx, sy, sz);
+  auto load = [&]() {
+    if (wave == 0) TileFeatures<0>::load(a, p, u, rho);
+    else if (wave == 1) TileFeatures<1>::load(a, p, u, rho);
+    else if (wave == 2) TileFeatures<2>::load(a, p, u, rho);
+    else TileFeatures<3>::load(a, p, u, rho);
+  };
+  auto put = [&](int buf) {
+    float gm;
+    if (wave == 0) gm = TileFeatures<0>::put(nrm, u, As, lane);
+    else if (wave == 1) gm = TileFeatures<1>::put(nrm, u, As, lane);
+    else if (wave == 2) gm = TileFeatures<2>::put(nrm, u, As, lane);
+    else gm = TileFeatures<3>::put(nrm, u, As, lane);
+    gms[buf][wave][lane] = gm;
+    if (wave == 0) rhos[buf][lane] = rho;
+  };
+  f32x4 acc[4];
+  auto product = [&](const uint2 (*src)[FT], const bf16x4 *w, int nkb) {
 #pragma unroll
-          for (int k = 0; k < 7; ++k) {
-            const int q = 243 + k;
-            const float v = (cell(c_sgs_tnb[k][0], c_sgs_tnb[k][1], c_sgs_tnb[k][2])[9] - smu[q]) * sisd[q];
-            gm = fmaxf(gm, fabsf(v));
-            row[q] = f2bf(v);
-          }
+    for (int rb = 0; rb < 4; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int q = SGS_NIN; q < SGS_KIN; ++q) row[q] = 0;
-        }
-      } else {
-        for (int q = p; q < SGS_KIN; q += 4) row[q] = 0;
-      }
-      gm = fmaxf(gm, __shfl_xor(gm, 1));
-      gm = fmaxf(gm, __shfl_xor(gm, 2));
-      if (p == 0) gms[r] = gm;
+    for (int kb = 0; kb < nkb; ++kb) {
+      if (kb > 0 && kb % 4 == 0) __builtin_amdgcn_sched_barrier(0);   /* 16 operand reads in flight, no more registers */
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w[kb], ld_frag(&src[4 * kb + lk][16 * rb + lr]), acc[rb], 0, 0, 0);
     }
+  };
+  auto store_act = [&](int buf, int layer) {
+    const float4 b4 = *(const float4 *)&cf[layer][16 * wave + 4 * lk];
+    const float b[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+      Hs[buf][4 * wave + lk][16 * rb + lr] = make_uint2(f2bf2(gelu(acc[rb][0] + b[0]), gelu(acc[rb][1] + b[1])),
+                                                        f2bf2(gelu(acc[rb][2] + b[2]), gelu(acc[rb][3] + b[3])));
+  };
+  unsigned ncnt = 0, npass = 0;          /* cells finished and passing, by lanes 0..15 of each wave */
+  int buf = 0;
+  if ((int)blockIdx.x < a.ntiles) {
+    load();
+    __syncthreads();                     /* nrm, cf */
+    put(0);
+  }
+  for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x, buf ^= 1) {
+    const int next = tile + gridDim.x;
     __syncthreads();
-    /* ---- layers 1-3: wave w computes the 64 x 16 column block w ---- */
-    f32x4 acc[4];
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < 16; ++kb)
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ld_frag(&As[16 * rb + lr][16 * kb + 4 * lk]), w1[kb], acc[rb], 0, 0, 0);
-    auto store_act = [&](int buf, float b) {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Hs[buf][16 * rb + 4 * lk + v][ncol] = f2bf(gelu(acc[rb][v] + b));
-    };
-    store_act(0, b1);
+    if (next < a.ntiles) {
+      p.advance(a, step, sx, sy, sz);
+      load();
+    }
+    product(As, w1, 16);
+    store_act(0, 0);
     __syncthreads();
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (next < a.ntiles) put(buf ^ 1);
+    product(Hs[0], w2, 4);
+    store_act(1, 1);
+    __syncthreads();
+    product(Hs[1], w3, 4);
+    store_act(0, 2);
+    __syncthreads();
+    /* ---- layer 4 and finish: wave w the cell block w, the lane's outputs 4 lk .. 4 lk + 3 ---- */
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
+      o = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w4[kb], ld_frag(&Hs[0][4 * kb + lk][16 * wave + lr]), o, 0, 0, 0);
+    const int r = 16 * wave + lr;
+    const long c = (long)tile * FT + r;
+    const float rc = rhos[buf][r];
+    float t[4];
+    const float *b4 = &cf[3][4 * lk], *ysd = b4 + SGS_KOUT, *ymu = ysd + SGS_KOUT;
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ld_frag(&Hs[0][16 * rb + lr][16 * kb + 4 * lk]), w2[kb], acc[rb], 0, 0, 0);
-    store_act(1, b2);
-    __syncthreads();
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ld_frag(&Hs[1][16 * rb + lr][16 * kb + 4 * lk]), w3[kb], acc[rb], 0, 0, 0);
-    store_act(0, b3);
-    __syncthreads();
-    /* ---- layer 4: wave w the row block w ---- */
-    {
-      f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-        o = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ld_frag(&Hs[0][16 * wave + lr][16 * kb + 4 * lk]), w4[kb], o, 0, 0, 0);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) Ys[16 * wave + 4 * lk + v][lr] = o[v] + b4;
+    for (int v = 0; v < 4; ++v) {
+      const float y = o[v] + b4[v];
+      t[v] = y * ysd[v] + ymu[v];
     }
-    __syncthreads();
-    /* ---- finish ---- */
-    if (tid < FT) {
-      const long c = c0 + tid;
-      if (c < a.ncell) {
-        int x, y, z;
-        cell_xyz(c, a.Nx, a.Ny, x, y, z);
-        const float rho = a.S[(long)z * a.ps + (long)y * a.P + x];
-        npass += sgs_finish_cell(Ys[tid], a.ymu, a.ysd, gms[tid], a.gate, rho, c, a.tauL, a.ncell, a.mask) ? 1u : 0u;
+    const float t4 = __shfl_down(t[0], 16), t5 = __shfl_down(t[1], 16);
+    if (c < a.ncell) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (4 * lk + v < SGS_NOUT) a.tauL[(4 * lk + v) * a.ncell + c] = rc * t[v];
+      if (lk == 0) {
+        const float gm = fmaxf(fmaxf(gms[buf][0][r], gms[buf][1][r]), fmaxf(gms[buf][2][r], gms[buf][3][r]));
+        const bool ok = gm <= a.gate && sgs_realizable(t[0], t[1], t[2], t[3], t4, t5);
+        a.mask[c] = ok ? 1 : 0;
+        npass += ok ? 1u : 0u;
         ++ncnt;
       }
     }
-    __syncthreads();
   }
-  /* one pair of atomics per work-group (wave 0 holds every finishing thread) */
-  if (wave == 0) {
+  /* one pair of atomics per work-group */
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      ncnt += __shfl_xor(ncnt, off);
-      npass += __shfl_xor(npass, off);
-    }
-    if (lane == 0 && ncnt) {
-      atomicAdd(&a.count[0], (unsigned long long)ncnt);
-      atomicAdd(&a.count[1], (unsigned long long)npass);
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    ncnt += __shfl_xor(ncnt, off);
+    npass += __shfl_xor(npass, off);
+  }
+  if (lane == 0) {
+    cnts[wave][0] = ncnt;
+    cnts[wave][1] = npass;
+  }
+  __syncthreads();
+  if (tid == 0 && (int)blockIdx.x < a.ntiles) {
+    atomicAdd(&a.count[0], (unsigned long long)(cnts[0][0] + cnts[1][0] + cnts[2][0] + cnts[3][0]));
+    atomicAdd(&a.count[1], (unsigned long long)(cnts[0][1] + cnts[1][1] + cnts[2][1] + cnts[3][1]));
   }
 }
 
