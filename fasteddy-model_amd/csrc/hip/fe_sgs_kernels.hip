@@ -342,7 +342,8 @@ __global__ void __launch_bounds__(256) k_sgs_features(FeatArgs a) {
 }
 
 /* Gradient pass of the fused inference: one thread per cell of [c0, c0 + nc), the ten values
- * of sgs_grad_cell into G[cell][12] (the last two padding). */
+ * of sgs_grad_cell into G: [cells][4], [cells][4], [cells], [cells] (a wave's gathers there are
+ * contiguous; in records of 12 floats a cell each spread over three times the lines). */
 __global__ void __launch_bounds__(256) k_sgs_grad(FeatArgs a, float *G) {
   const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= a.nc) return;
@@ -351,10 +352,11 @@ __global__ void __launch_bounds__(256) k_sgs_grad(FeatArgs a, float *G) {
   cell_xyz(c, a.Nx, a.Ny, x, y, z);
   float g[10];
   sgs_grad_cell(a, x, y, z, g);
-  float4 *o = (float4 *)(G + c * 12);
-  o[0] = make_float4(g[0], g[1], g[2], g[3]);
-  o[1] = make_float4(g[4], g[5], g[6], g[7]);
-  o[2] = make_float4(g[8], g[9], 0.f, 0.f);
+  const long n = (long)a.Nx * a.Ny * a.Nz;
+  ((float4 *)G)[c] = make_float4(g[0], g[1], g[2], g[3]);
+  ((float4 *)(G + 4 * n))[c] = make_float4(g[4], g[5], g[6], g[7]);
+  G[8 * n + c] = g[8];
+  G[9 * n + c] = g[9];
 }
 
 /* ---- training data: box filter of a fine state ------------------------------------------- */
@@ -476,14 +478,16 @@ __global__ void k_sgs_finish(const float *Y, const float *ymu, const float *ysd,
  * increasing order, FP32 bias and GELU) are those of the unfused kernels, so both paths give
  * the same bits.
  * What bounds it: vector instructions, 970 per wave and tile (600 of them the GELUs), at two waves
- * per SIMD (the prefetched features and the weights are 128 registers).
+ * per SIMD (the prefetched features and the weights are 128 registers), then its gathers.
  * 128 x 128 x 48: 234 us with four lanes per cell that read each feature's normalisation from LDS,
  * stored it as two bytes and waited for every neighbour's loads, and a serial finish by one wave;
- * 169 us so.  A contiguous run of tiles per XCD made no difference (170 us). */
+ * 170 us without, 164 us with the gradients by component (k_sgs_grad) instead of in records of 12
+ * floats.  A contiguous run of tiles per XCD made no difference (170 us), nor did scalar
+ * normalisation operands; chaining the layers in registers, a wave per 16 cells, was slower (180 us). */
 constexpr int FT = 64;
 
 struct FusedArgs {
-  const float *G;                        /* [cells][12] from k_sgs_grad */
+  const float *G;                        /* gradients from k_sgs_grad */
   int Nx, Ny, Nz;
   const float *mu, *isd;                 /* feature normalisation [256] */
   const float *w;                        /* FP32 master parameters */
@@ -538,29 +542,32 @@ struct TileFeatures {
     if (W == 0) rho = a.S[(long)p.z * a.ps + (long)p.y * a.P + p.x];
     /* a neighbour's place is the cell's plus one step per direction, wrapped or clamped by the step
      * (32 bits, modulo 2^32: the sum is a place in the grid) */
-    const unsigned c12 = 12u * (unsigned)p.c, row = 12u * (unsigned)a.Nx, plane = row * (unsigned)a.Ny;
-    const unsigned xo[3] = {p.x == 0 ? row - 12u : -12u, 0u, p.x == a.Nx - 1 ? 12u - row : 12u};
+    const unsigned c = (unsigned)p.c, row = (unsigned)a.Nx, plane = row * (unsigned)a.Ny;
+    const unsigned xo[3] = {p.x == 0 ? row - 1u : -1u, 0u, p.x == a.Nx - 1 ? 1u - row : 1u};
     const unsigned yo[3] = {p.y == 0 ? plane - row : -row, 0u, p.y == a.Ny - 1 ? row - plane : row};
     const unsigned zo[3] = {p.z == 0 ? 0u : -plane, 0u, p.z == a.Nz - 1 ? 0u : plane};
-    auto cell = [&](int dx, int dy, int dz) -> const float * { return a.G + (c12 + zo[dz + 1] + yo[dy + 1] + xo[dx + 1]); };
+    auto cell = [&](int dx, int dy, int dz) -> unsigned { return c + zo[dz + 1] + yo[dy + 1] + xo[dx + 1]; };
+    const float4 *ga = (const float4 *)a.G, *gb = (const float4 *)(a.G + 4 * a.ncell);
+    const float *gc = a.G + 8 * a.ncell;
 #pragma unroll
     for (int i = 0; i < NN; ++i) {
       const int n = N0 + i;
-      const float4 *g4 = (const float4 *)cell(n % 3 - 1, (n / 3) % 3 - 1, n / 9 - 1);
-      const float4 u0 = g4[0], u1 = g4[1];
+      const unsigned id = cell(n % 3 - 1, (n / 3) % 3 - 1, n / 9 - 1);
+      const float4 u0 = ga[id], u1 = gb[id];
       u[9 * i + 0] = u0.x; u[9 * i + 1] = u0.y; u[9 * i + 2] = u0.z; u[9 * i + 3] = u0.w;
       u[9 * i + 4] = u1.x; u[9 * i + 5] = u1.y; u[9 * i + 6] = u1.z; u[9 * i + 7] = u1.w;
-      u[9 * i + 8] = ((const float *)g4)[8];
+      u[9 * i + 8] = gc[id];
     }
     if constexpr (W == 3) {
       /* dtheta/dz of the cell, x-, x+, y-, y+, z-, z+ (c_sgs_tnb) */
-      u[TH + 0] = cell(0, 0, 0)[9];
-      u[TH + 1] = cell(-1, 0, 0)[9];
-      u[TH + 2] = cell(1, 0, 0)[9];
-      u[TH + 3] = cell(0, -1, 0)[9];
-      u[TH + 4] = cell(0, 1, 0)[9];
-      u[TH + 5] = cell(0, 0, -1)[9];
-      u[TH + 6] = cell(0, 0, 1)[9];
+      const float *gt = gc + a.ncell;
+      u[TH + 0] = gt[cell(0, 0, 0)];
+      u[TH + 1] = gt[cell(-1, 0, 0)];
+      u[TH + 2] = gt[cell(1, 0, 0)];
+      u[TH + 3] = gt[cell(0, -1, 0)];
+      u[TH + 4] = gt[cell(0, 1, 0)];
+      u[TH + 5] = gt[cell(0, 0, -1)];
+      u[TH + 6] = gt[cell(0, 0, 1)];
       /* the same last element in every wave's branch: the array stays in registers */
 #pragma unroll
       for (int i = TH + 7; i < 72; ++i) u[i] = 0.f;
