@@ -301,17 +301,23 @@ Variant make_variant(const char *name) {
   return v;
 }
 
+Variant g_var;      /* the model's kernels, for any blending weights */
+Variant g_var_sb;   /* the same for one weight of every field; g_var where the schemes have no weight to share */
+int g_var_ok = 0;
+
 template <bool TKE, int NM, int SH, int SE, int SQV, int SQL, bool ENS = false, bool TERR = false>
-Variant pick_variant(const char *name) {
+void set_variants(const char *name) {
+  g_var = g_var_sb = make_variant<TKE, NM, SH, SE, SQV, SQL, ENS, TERR, false>(name);
   constexpr bool hyb = SH == 2 || SH == 3;                 /* schemes with a blending weight */
-  const bool sb = (!TKE || b_hyb == TKEAdvSelector_b_hyb) && (NM == 0 || b_hyb == moistureAdvSelectorQv_b);
-  if constexpr (hyb && (TKE || NM > 0))
-    if (sb) return make_variant<TKE, NM, SH, SE, SQV, SQL, ENS, TERR, true>(name);
-  return make_variant<TKE, NM, SH, SE, SQV, SQL, ENS, TERR, false>(name);
+  if constexpr (hyb && (TKE || NM > 0)) g_var_sb = make_variant<TKE, NM, SH, SE, SQV, SQL, ENS, TERR, true>(name);
 }
 
-Variant g_var;
-int g_var_ok = 0;
+/* The kernels for the weights that a launch carries: they are the program's variables, read for every
+ * launch (for an ensemble member when it is added), and need not be those of the set-up. */
+const Variant &variant_of(const StepArgs &a) {
+  const bool one = (D.nTKE == 0 || a.be == a.bh) && (D.nM == 0 || a.bqv == a.bh);
+  return one ? g_var_sb : g_var;
+}
 
 int select_variant(void) {
   const int tke = (turbulenceSelector > 0 && TKESelector > 0);
@@ -325,11 +331,11 @@ int select_variant(void) {
      * advection with the prognostic-TKE closure (dry, and the shallow-cumulus q_v/q_l set with
      * WENO5 liquid) and with the Smagorinsky closure (dry) */
     if (tke && nm == 0 && sh == 3 && se == 3) {
-      g_var = pick_variant<true, 0, 3, 3, 3, 5, false, true>("dry+tke hyb56/hyb56 terrain-following");
+      set_variants<true, 0, 3, 3, 3, 5, false, true>("dry+tke hyb56/hyb56 terrain-following");
     } else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 5) {
-      g_var = pick_variant<true, 2, 3, 3, 3, 5, false, true>("moist2+tke hyb56/hyb56/hyb56/weno5 terrain-following");
+      set_variants<true, 2, 3, 3, 3, 5, false, true>("moist2+tke hyb56/hyb56/hyb56/weno5 terrain-following");
     } else if (!tke && turbulenceSelector > 0 && nm == 0 && sh == 3) {
-      g_var = pick_variant<false, 0, 3, 3, 3, 5, false, true>("dry smagorinsky hyb56 terrain-following");
+      set_variants<false, 0, 3, 3, 3, 5, false, true>("dry smagorinsky hyb56 terrain-following");
     } else {
       fprintf(stderr, "select_variant: terrain-following grids run HYB56 advection with the prognostic-TKE closure "
                       "(dry, or q_v/q_l with WENO5 liquid) or the dry Smagorinsky closure\n");
@@ -338,21 +344,21 @@ int select_variant(void) {
     g_var_ok = 1;
     return FE_OK;
   }
-  if (tke && nm == 0 && sh == 3 && se == 3) { g_var = pick_variant<true, 0, 3, 3, 3, 5, true>("dry+tke hyb56/hyb56"); g_var_ok = 1; }
-  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 5) { g_var = pick_variant<true, 2, 3, 3, 3, 5, true>("moist2+tke hyb56/hyb56/hyb56/weno5"); g_var_ok = 1; }
-  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 2 && sql == 5) { g_var = pick_variant<true, 2, 3, 3, 2, 5>("moist2+tke hyb56/hyb56/hyb34/weno5"); g_var_ok = 1; }
-  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 0) { g_var = pick_variant<true, 2, 3, 3, 3, 0>("moist2+tke hyb56/.../upstream"); g_var_ok = 1; }
-  else if (tke && nm == 1 && sh == 3 && se == 3 && sqv == 3) { g_var = pick_variant<true, 1, 3, 3, 3, 5>("moist1+tke hyb56"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 5 && se == 5) { g_var = pick_variant<true, 0, 5, 5, 3, 5>("dry+tke weno5/weno5"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 2 && se == 2) { g_var = pick_variant<true, 0, 2, 2, 3, 5>("dry+tke hyb34/hyb34"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 1 && se == 1) { g_var = pick_variant<true, 0, 1, 1, 3, 5>("dry+tke quick/quick"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 0 && se == 0) { g_var = pick_variant<true, 0, 0, 0, 3, 5>("dry+tke upstream"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 6 && se == 6) { g_var = pick_variant<true, 0, 6, 6, 3, 5>("dry+tke centred2"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 4 && se == 4) { g_var = pick_variant<true, 0, 4, 4, 3, 5>("dry+tke weno3"); g_var_ok = 1; }
-  else if (tke && nm == 0 && sh == 3 && se == 0) { g_var = pick_variant<true, 0, 3, 0, 3, 5>("dry+tke hyb56/upstream"); g_var_ok = 1; }
-  else if (!tke && turbulenceSelector == 0 && nm == 0 && sh == 3) { g_var = pick_variant<false, 0, 3, 3, 3, 5>("dry inviscid hyb56"); g_var_ok = 1; }
-  else if (!tke && turbulenceSelector > 0 && nm == 0 && sh == 3) { g_var = pick_variant<false, 0, 3, 3, 3, 5, true>("dry smagorinsky hyb56"); g_var_ok = 1; }
-  else if (!tke && turbulenceSelector > 0 && nm == 2 && sh == 3 && sqv == 3 && sql == 5) { g_var = pick_variant<false, 2, 3, 3, 3, 5>("moist2 smagorinsky hyb56/hyb56/weno5"); g_var_ok = 1; }
+  if (tke && nm == 0 && sh == 3 && se == 3) { set_variants<true, 0, 3, 3, 3, 5, true>("dry+tke hyb56/hyb56"); g_var_ok = 1; }
+  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 5) { set_variants<true, 2, 3, 3, 3, 5, true>("moist2+tke hyb56/hyb56/hyb56/weno5"); g_var_ok = 1; }
+  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 2 && sql == 5) { set_variants<true, 2, 3, 3, 2, 5>("moist2+tke hyb56/hyb56/hyb34/weno5"); g_var_ok = 1; }
+  else if (tke && nm == 2 && sh == 3 && se == 3 && sqv == 3 && sql == 0) { set_variants<true, 2, 3, 3, 3, 0>("moist2+tke hyb56/.../upstream"); g_var_ok = 1; }
+  else if (tke && nm == 1 && sh == 3 && se == 3 && sqv == 3) { set_variants<true, 1, 3, 3, 3, 5>("moist1+tke hyb56"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 5 && se == 5) { set_variants<true, 0, 5, 5, 3, 5>("dry+tke weno5/weno5"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 2 && se == 2) { set_variants<true, 0, 2, 2, 3, 5>("dry+tke hyb34/hyb34"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 1 && se == 1) { set_variants<true, 0, 1, 1, 3, 5>("dry+tke quick/quick"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 0 && se == 0) { set_variants<true, 0, 0, 0, 3, 5>("dry+tke upstream"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 6 && se == 6) { set_variants<true, 0, 6, 6, 3, 5>("dry+tke centred2"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 4 && se == 4) { set_variants<true, 0, 4, 4, 3, 5>("dry+tke weno3"); g_var_ok = 1; }
+  else if (tke && nm == 0 && sh == 3 && se == 0) { set_variants<true, 0, 3, 0, 3, 5>("dry+tke hyb56/upstream"); g_var_ok = 1; }
+  else if (!tke && turbulenceSelector == 0 && nm == 0 && sh == 3) { set_variants<false, 0, 3, 3, 3, 5>("dry inviscid hyb56"); g_var_ok = 1; }
+  else if (!tke && turbulenceSelector > 0 && nm == 0 && sh == 3) { set_variants<false, 0, 3, 3, 3, 5, true>("dry smagorinsky hyb56"); g_var_ok = 1; }
+  else if (!tke && turbulenceSelector > 0 && nm == 2 && sh == 3 && sqv == 3 && sql == 5) { set_variants<false, 2, 3, 3, 3, 5>("moist2 smagorinsky hyb56/hyb56/weno5"); g_var_ok = 1; }
   return g_var_ok ? FE_OK : FE_ERR_UNSUPPORTED;
 }
 
@@ -477,6 +483,7 @@ void halo_fill(float *S, long fs, int nf, int nz) {
 int launch_stage(int stage, const float *in, const float *base, float *out, int emitF, float *pout) {
   StepArgs a;
   fill_args(a, stage, in, base, out, emitF, pout);
+  const Variant &var = variant_of(a);
   /* the stage reads its input's lateral halo (the exchange of a decomposed run) */
   if (D.halo) halo_fill(const_cast<float *>(in), D.fs, D.NF, D.Nz);
   const int phys = physics_stage(stage) && turbulenceSelector > 0;
@@ -493,15 +500,15 @@ int launch_stage(int stage, const float *in, const float *base, float *out, int 
     const int ext = D.halo ? 2 : 0;
     if (D.halo) halo_fill(D.surf, D.ps, SF_N, 1);
     dim3 cg((D.Nx + ext + 255) / 256, D.Ny + ext);
-    launch_timed(0, g_var.surface, cg, dim3(256), a);
+    launch_timed(0, var.surface, cg, dim3(256), a);
   }
   dim3 grid((D.Nx + TX - 1) / TX, (D.Ny + TY - 1) / TY, D.nseg);
   /* the batch's last stage also emits the SGS stresses and tendencies the host will read */
   const bool emit = a.tau || a.mtau || a.fem;
   /* the microphysics runs every few steps (a.mpActive); the steps between use the physics
    * kernel compiled without it, which has the registers to spare (no spill when moist) */
-  stage_fn k = phys ? (emit ? g_var.phys_emit : (a.mpActive ? g_var.phys : g_var.phys_nomp))
-                    : (emit ? g_var.plain_emit : g_var.plain);
+  stage_fn k = phys ? (emit ? var.phys_emit : (a.mpActive ? var.phys : var.phys_nomp))
+                    : (emit ? var.plain_emit : var.plain);
   launch_timed(phys ? 2 : 1, k, grid, dim3(NT), a);
   HIPCHK(hipGetLastError());
   if (learned) return sgs_correct(out, emitF ? 1.f : a.coefdt);

@@ -353,7 +353,6 @@ int fe_ens_add_member(void) {
         fprintf(stderr, "fe_ens_add_member: members must share the physics-stage schedule (physics_oneRKonly)\n");
         return -FE_ERR_UNSUPPORTED;
       }
-    if (E.var.sb && !g_var.sb) E.var = g_var;    /* a member whose blending weights differ: kernels for any weights */
   } else {
     E.var = g_var;
     E.have_var = true;
@@ -373,6 +372,8 @@ int fe_ens_add_member(void) {
   fill_args(m.args[0], 0, m.S[0], m.S[0], m.S[1], 0, nullptr);
   fill_args(m.args[1], 1, m.S[1], m.S[0], m.S[2], 0, nullptr);
   fill_args(m.args[2], 2, m.S[2], m.S[0], m.S[0], 0, nullptr);
+  const Variant &var = variant_of(m.args[0]);
+  if (E.mem.empty() || E.var.sb) E.var = var;    /* kernels for any weights once a member's weights differ */
   m.mptf = 0;
   if (moistureSelector > 0 && moistureCond > 0 && moistureNvars > 1)
     m.mptf = (int)roundf(fmaxf(moistureMPcallTscale, dt) / dt);
