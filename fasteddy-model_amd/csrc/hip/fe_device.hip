@@ -120,6 +120,7 @@ struct Dev {
 
 }  // namespace
 
+#include "fe_segments.h"
 #include "fe_transfer.hip"
 
 namespace {
@@ -412,17 +413,6 @@ void fill_args(StepArgs &a, int stage, const float *in, const float *base, float
 
 inline int physics_stage(int stage) { return (physics_oneRKonly == 0) || (stage == numRKstages); }
 
-/* Split the column into z segments, one work-group per tile and segment, when the
- * tiles alone leave compute units idle: a stage work-group holds one compute unit
- * (its LDS), so fewer than 256 tiles (e.g. 256 x 256 cells = 128 tiles) would run
- * the chip at tiles/256.  Segments are even; amd_zSegments > 0 sets the count. */
-/* Even segment length for n segments of Nz levels, and the segment count it gives. */
-static void seg_shape(int Nz, int n, int &len, int &nseg) {
-  len = (Nz + n - 1) / n;
-  len += len & 1;
-  nseg = (Nz + len - 1) / len;
-}
-
 /* Work-groups of a stage launch that run at once on one compute unit (LDS and registers
  * decide: one on the 64 x 8 tile, two on the 16 x 16 tile), the lower of the variant's
  * two stage kernels. */
@@ -434,7 +424,11 @@ static int stage_wg_per_cu(const Variant &v) {
   return std::max(1, std::min(o1, o2));
 }
 
-/* A launch runs in rounds of (work-groups per CU) x CUs work-groups; a segment also loads its
+/* Split the column into z segments, one work-group per tile and segment, when the
+ * tiles alone leave compute units idle: a stage work-group holds one compute unit
+ * (its LDS), so fewer than 256 tiles (e.g. 256 x 256 cells = 128 tiles) would run
+ * the chip at tiles/256.  Segments are even; amd_zSegments > 0 sets the count.
+ * A launch runs in rounds of (work-groups per CU) x CUs work-groups; a segment also loads its
  * window and fills its pipeline (about 2 levels' worth of set-up).  The count minimises rounds x
  * (segment length + 2) over segments of at least 4 levels (fewest segments on ties): a count
  * whose work-groups overflow the slots by a few would add a nearly empty round, and a small grid

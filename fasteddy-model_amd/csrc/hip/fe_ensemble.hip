@@ -92,49 +92,16 @@ int ens_slots() {
   return ncu * occ;
 }
 
-/* Levels' worth of a work item: its levels and about two for loading its window and filling the
- * pipeline. */
-inline int ens_item_cost(int levels) { return levels + 2; }
-
-/* Segments of the members that have none set: the segment length, of all even lengths >= 4, whose
- * work items end earliest when the work-groups of the persistent grid take them longest first
- * (longest length on ties).  A lone run's own choice spreads one member over the whole chip; here
- * the members fill it together, and segments as short as a lone 64 x 64 x 48 member's (4 levels)
- * spend a third of their items on set-up.  Measured in ms a step, lone-run choice -> this one: 16 of
- * 64 x 64 x 48 0.399 (12 segments) -> 0.335 (2); 40 of them 0.928 -> 0.765 (4); eight of 96^2 x 64 to
- * 192^2 x 96 within 1% of the best length of 8, 12, 16, 24, 32, 48, 64 levels, 48 of them within 3%. */
+/* Segments of the members that have none set, chosen for all members together. */
 void ens_default_segments() {
   if (!E.seg_old) return;
   E.seg_old = false;
-  const int slots = ens_slots();
-  int mz = 0;
+  std::vector<SegMember> mem;
   for (auto &m : E.mem)
-    if (!m.seg_set) mz = std::max(mz, m.Nz);
-  long best = -1;
-  int blen = 0;
-  for (int len = 4; len < mz + 2; len += 2) {
-    std::map<int, long, std::greater<int>> items;      /* item cost -> items */
-    for (auto &m : E.mem) {
-      const long tiles = (long)((m.Nx + TX - 1) / TX) * ((m.Ny + TY - 1) / TY);
-      int zseg = m.zseg, nseg = m.nseg;
-      if (!m.seg_set) seg_shape(m.Nz, (m.Nz + len - 1) / len, zseg, nseg);
-      items[ens_item_cost(std::min(zseg, m.Nz))] += tiles * (nseg - 1);
-      items[ens_item_cost(m.Nz - (nseg - 1) * zseg)] += tiles;
-    }
-    std::map<long, long> load{{0, slots}};              /* work taken -> work-groups */
-    for (auto &it : items)
-      for (long left = it.second; left > 0;) {
-        const auto lo = load.begin();
-        const long at = lo->first, n = std::min(left, lo->second);
-        if ((lo->second -= n) == 0) load.erase(lo);
-        load[at + it.first] += n;
-        left -= n;
-      }
-    const long end = load.rbegin()->first;
-    if (best < 0 || end <= best) { best = end; blen = len; }
-  }
+    mem.push_back(SegMember{(long)((m.Nx + TX - 1) / TX) * ((m.Ny + TY - 1) / TY), m.Nz, m.seg_set ? m.zseg : 0});
+  const int len = ens_segment_length(mem, ens_slots());
   for (auto &m : E.mem)
-    if (!m.seg_set) ens_set_segments(m, (m.Nz + blen - 1) / blen);
+    if (!m.seg_set) ens_set_segments(m, (m.Nz + len - 1) / len);
 }
 
 int ens_drop_graph() {
