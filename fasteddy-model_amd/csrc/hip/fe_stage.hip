@@ -266,6 +266,12 @@ struct Cfg {
   static constexpr int IE_SAFE = TKE_ ? IE : 0;
   static constexpr int SH = SH_, SE = SE_, SQV = SQV_, SQL = SQL_;
   static constexpr bool PHYS = PHYS_;
+  /* own cell and x fluxes in registers (own_faces); through LDS (own_faces_lds) where the kernel has
+   * no registers left for them.  256 x 256 x 160, us a launch, registers -> LDS: moist over a hill
+   * plain stage 500 (29 VGPRs spilled) -> 383 (none), physics stage 722 (24) -> 692 (20); dry WENO5
+   * plain stage 584 (21) -> 465 (none).  Nothing spills and registers are faster in the WENO5 physics
+   * stage (528, LDS 556) and in the others (dry plain 192, LDS 255; moist flat plain 310, LDS 321). */
+  static constexpr bool REG = !(NM_ > 0 && TERR_) && (PHYS_ || SH_ != 5);
   static constexpr int NV = 4 + NM_;          /* u, v, w, theta, q/rho ... */
   static constexpr int NB = 4 + NM_;          /* face stress components per face family */
   template <int F> static constexpr int sch() {
@@ -293,19 +299,33 @@ __device__ __forceinline__ float lane_up(float v, float edge, int tx) {
   if constexpr (TX == 64) return __builtin_bit_cast(float, r);
   else return tx == TX - 1 ? edge : __builtin_bit_cast(float, r);
 }
+/* x fluxes in LDS: those of the ring column x = TX (16-byte rows), or of every face of the tile */
+template <class C, bool REG = C::REG>
+struct XFaces {
+  float g[TY][NFP];
+  __device__ __forceinline__ float &at(int f, int fy, int) { return g[fy][f]; }
+};
+template <class C>
+struct XFaces<C, false> {
+  float g[C::NF][TY][TX + 1];
+  __device__ __forceinline__ float &at(int f, int fy, int fx) { return g[f][fy][fx]; }
+};
 template <class C, int F, int FE = C::NF>
 struct FaceLoop {
-  /* x face fx = TX of row fy (the tile's ring column) */
-  __device__ __forceinline__ static void xr(float (*raw)[RH][RW], float *g, int fy, float U, const float *omb) {
+  __device__ __forceinline__ static void xf(float (*raw)[RH][RW], XFaces<C> &gx, int fy, int fx, float U, const float *omb) {
     if constexpr (F < FE) {
-      const SRD *r = lds_at<F * RH * RW>((const SRD *)&raw[0][fy + HH][TX]);
-      g[F] = face_flux<C::template sch<F>(), C::PHYS>(U, omb[F], r[0], r[1], r[2], r[3], r[4], r[5]);
-      FaceLoop<C, F + 1, FE>::xr(raw, g, fy, U, omb);
+      const SRD *o = (const SRD *)&raw[0][fy + HH][fx], *r;
+      if constexpr (C::REG) r = lds_at<F * RH * RW>(o);
+      else r = o + F * RH * RW;
+      gx.at(F, fy, fx) = face_flux<C::template sch<F>(), C::PHYS>(U, omb[F], r[0], r[1], r[2], r[3], r[4], r[5]);
+      FaceLoop<C, F + 1, FE>::xf(raw, gx, fy, fx, U, omb);
     }
   }
   __device__ __forceinline__ static void yf(float (*raw)[RH][RW], float (*gy)[TY + 1][TX], int fy, int fx, float V, const float *omb) {
     if constexpr (F < FE) {
-      const SRD *o = (const SRD *)&raw[0][fy][fx + HH], *r = lds_at<F * RH * RW>(o);
+      const SRD *o = (const SRD *)&raw[0][fy][fx + HH], *r;
+      if constexpr (C::REG) r = lds_at<F * RH * RW>(o);
+      else r = o + F * RH * RW;
       gy[F][fy][fx] = face_flux<C::template sch<F>(), C::PHYS>(V, omb[F], r[0], r[RW], r[2 * RW], r[3 * RW],
                                                                o[F * RH * RW + 4 * RW], o[F * RH * RW + 5 * RW]);
       FaceLoop<C, F + 1, FE>::yf(raw, gy, fy, fx, V, omb);
@@ -377,6 +397,16 @@ __device__ __forceinline__ void own_faces(float (*raw)[RH][RW], const float (*dr
   }
 }
 
+/* The same through LDS (C::REG off): the own cell read there as its neighbours are, fluxes to gx and gy. */
+template <class C>
+__device__ __forceinline__ void own_faces_lds(float (*raw)[RH][RW], const float (*dr)[DW], int ty, int tx, float hxD, float hyD,
+                                              const float *omb, XFaces<C> &gx, float (*gy)[TY + 1][TX]) {
+  const float U = hxD * (raw[1][ty + HH][tx + HH - 1] * dr[ty + 1][tx] + raw[1][ty + HH][tx + HH] * dr[ty + 1][tx + 1]);
+  FaceLoop<C, 0>::xf(raw, gx, ty, tx, U, omb);
+  const float V = hyD * (raw[2][ty + HH - 1][tx + HH] * dr[ty][tx + 1] + raw[2][ty + HH][tx + HH] * dr[ty + 1][tx + 1]);
+  FaceLoop<C, 0>::yf(raw, gy, ty, tx, V, omb);
+}
+
 /* Advective fluxes of fields [F0, F1) through the tile's ring faces: face i of the y face
  * row y = TY and face i of the x face column x = TX. */
 template <class C, int F0, int F1>
@@ -387,11 +417,11 @@ __device__ __forceinline__ void ring_faces_y(float (*raw)[RH][RW], float (*gy)[T
   FaceLoop<C, F0, F1>::yf(raw, gy, fy, fx, V, omb);
 }
 template <class C, int F0, int F1>
-__device__ __forceinline__ void ring_faces_x(float (*raw)[RH][RW], float (*gxr)[NFP], const float (*dr)[DW], int i,
+__device__ __forceinline__ void ring_faces_x(float (*raw)[RH][RW], XFaces<C> &gx, const float (*dr)[DW], int i,
                                              float hxD, const float *omb) {
   const int fx = TX, fy = i;
   const float U = hxD * (raw[1][fy + HH][fx + HH - 1] * dr[fy + 1][fx] + raw[1][fy + HH][fx + HH] * dr[fy + 1][fx + 1]);
-  FaceLoop<C, F0, F1>::xr(raw, gxr[fy], fy, U, omb);
+  FaceLoop<C, F0, F1>::xf(raw, gx, fy, fx, U, omb);
 }
 
 /* SGS stress pieces on a face-located cell (cuda_sgsTurbDevice.cu:60-367).  All
@@ -854,7 +884,7 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
   __shared__ float raw[NF][RH][RW];
   __shared__ float dvr[DH][DW];          /* rho^-1 of the ring-1 region (terrain-following grids: D rho^-1) */
   __shared__ float dvp[DH][DW];
-  __shared__ __align__(16) float gxr[TY][NFP];      /* x fluxes of the ring column x = TX */
+  __shared__ __align__(16) XFaces<C> gx;
   __shared__ float gy[NF][TY + 1][TX];
   /* velocities u,v,w rotate over four levels, theta and moisture over three */
   __shared__ float velm[PH ? 4 : 1][PH ? 3 : 1][DH][DW];
@@ -1239,22 +1269,26 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
       const float (*dfv)[DW] = dvr;
       /* own x face (low face of the own cell) and own y face */
       {
-        float c[NF];
+        if constexpr (C::REG) {
+          float c[NF];
 #pragma unroll
-        for (int f = 0; f < NF; ++f) c[f] = win[f][3];
-        own_faces<C>(raw, dfv, ty, tx, c, C::TERR ? dfv[ty + 1][tx + 1] : rin, hxD, hyD, omb, fx, fy);
+          for (int f = 0; f < NF; ++f) c[f] = win[f][3];
+          own_faces<C>(raw, dfv, ty, tx, c, C::TERR ? dfv[ty + 1][tx + 1] : rin, hxD, hyD, omb, fx, fy);
 #pragma unroll
-        for (int f = 0; f < NF; ++f) gy[f][ty][tx] = fy[f];
+          for (int f = 0; f < NF; ++f) gy[f][ty][tx] = fy[f];
+        } else {
+          own_faces_lds<C>(raw, dfv, ty, tx, hxD, hyD, omb, gx, gy);
+        }
       }
       /* ring faces (on the 64 x 8 tile half of the fields per job row) */
       {
         constexpr int HF = PL.split ? NF / 2 : NF;
         int i;
         if (on_job(PL.rfy[0], wave, lane, i)) ring_faces_y<C, 0, HF>(raw, gy, dfv, i, hyD, omb);
-        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, HF>(raw, gxr, dfv, i, hxD, omb);
+        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, HF>(raw, gx, dfv, i, hxD, omb);
         if constexpr (PL.split) {
           if (on_job(PL.rfy[1], wave, lane, i)) ring_faces_y<C, HF, NF>(raw, gy, dfv, i, hyD, omb);
-          if (on_job(PL.rfx[1], wave, lane, i)) ring_faces_x<C, HF, NF>(raw, gxr, dfv, i, hxD, omb);
+          if (on_job(PL.rfx[1], wave, lane, i)) ring_faces_x<C, HF, NF>(raw, gx, dfv, i, hxD, omb);
         }
       }
       if constexpr (PH) {
@@ -1362,8 +1396,12 @@ __device__ __forceinline__ void stage_body(const StepArgs &a, TilePos tp) {
       const float rinp = frcp(win[0][4]);
       float dxy[NF], gzhi[NF], F[NF];
 #pragma unroll
-      for (int f = 0; f < NF; ++f)
-        dxy[f] = (lane_up(fx[f], ((const SRD *)gxr[ty])[f], tx) - fx[f]) + (((const SRD *)&gy[f][ty][tx])[TX] - fy[f]);
+      for (int f = 0; f < NF; ++f) {
+        if constexpr (C::REG)
+          dxy[f] = (lane_up(fx[f], ((const SRD *)gx.g[ty])[f], tx) - fx[f]) + (((const SRD *)&gy[f][ty][tx])[TX] - fy[f]);
+        else
+          dxy[f] = (gx.at(f, ty, tx + 1) - gx.at(f, ty, tx)) + (gy[f][ty + 1][tx] - gy[f][ty][tx]);
+      }
       dyn_tendency<C, 7>(a, z, C::TERR ? trow : dyn_rows<C>(a, z, (unsigned)col), win, rin, rinp, pz[0], pz[2], pgx, pgy, dxy,
                          gzlo, gzhi, omb, F);
       const float rho = win[0][3];
@@ -1563,14 +1601,15 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
   __shared__ float raw[2][NF][RH][RW];
   __shared__ float dvr[2][DH][DW];       /* rho^-1 of the ring-1 region (terrain-following grids: D rho^-1) */
   __shared__ float dvp[2][DH][DW];
-  __shared__ __align__(16) float gxr[2][TY][NFP];   /* x fluxes of the ring column x = TX */
+  __shared__ __align__(16) XFaces<C> gx[2];
   __shared__ float gy[2][NF][TY + 1][TX];
-  /* x fluxes through the own cells' low faces: carried in registers from P2 to the next
+  /* x fluxes through the own cells' low faces (C::REG): carried in registers from P2 to the next
    * iteration's P3, or through LDS when moist (two more fields, and no registers left) */
-  constexpr bool FXR = C::NM == 0;
-  /* RK base of P3's level loaded one iteration ahead, or (moist, for registers) at the start of its own */
-  constexpr bool BSA = C::NM == 0;
-  __shared__ float gxo[FXR ? 1 : 2][FXR ? 1 : NF][FXR ? 1 : TY][FXR ? 1 : TX];
+  constexpr bool FXR = C::REG && C::NM == 0, FXL = C::REG && !FXR;
+  /* RK base of P3's level loaded one iteration ahead, or (own cell in registers and moist, for
+   * registers) at the start of its own; moist over a hill 383 us a launch ahead, 397 at its own */
+  constexpr bool BSA = C::NM == 0 || !C::REG;
+  __shared__ float gxo[FXL ? 2 : 1][FXL ? NF : 1][FXL ? TY : 1][FXL ? TX : 1];
 
   constexpr RingPlan PL = PLAN_PLAIN;
   const Tile<C> T(a, tp, PL.r1);
@@ -1586,16 +1625,21 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
    *   hv[l+S]: halo cell, level it+l;  bs[S]: RK base of level it-2 (bs[S+1] in flight);
    *   pp[S..S+3]: own p' of levels it-3..it;  ri[S..S+2]: own rho^-1 of levels it-2..it;
    *   pg[S]: horizontal p' differences of level it-2 (pg[S+1] written for it-1);
-   *   gz: z flux through the lower face of level it-2;
+   *   gz[0]: z flux through the lower face of level it-2 (GZS: gz[S], gz[S+1] its upper face);
    *   fx[S]: x flux through the own cell's low face at level it-2 (fx[S+1] written for it-1). */
   /* The pipeline starts at the segment's first level it0 and computes no plane or face outside
    * [it0, ze): p' below the segment and the z flux through its lower face come from the set-up,
    * formed with the loop's own expressions (64 x 64 x 48 in 12 segments of 4 levels: six
    * iterations where two levels below the segment run without output made eight). */
   const int it0 = T.zs, ze = T.ze;
-  float gz[NF], pp[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+  /* the face's flux in slots that the rotation renames, or copied down in each iteration: WENO5 465 us
+   * in slots, 510 copied; moist over a hill 398 and 383 */
+  constexpr bool GZS = C::SH == 5;
+  float gz[GZS ? 3 : 1][NF], pp[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int f = 0; f < NF; ++f) gz[f] = 0.f;
+  for (int l = 0; l < (GZS ? 3 : 1); ++l)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) gz[l][f] = 0.f;
   /* from levels it0-3 .. it0+2: moist flat grids form it before the window is held (256 x 256 x 160:
    * 331 us after it, 307 before), the others from the window (terrain-following 256 x 256 x 128:
    * 227 us before, 215 from it; 64 x 64 x 48: 16.0 and 15.3) */
@@ -1603,7 +1647,7 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
     const float W = zface_vel(a, it0 - 1, cprof<C>(a, PR_D, it0 - 1, (unsigned)T.col), cprof<C>(a, PR_J33, it0 - 1, (unsigned)T.col),
                               w6[3][2], frcp(w6[0][2]), cprof<C>(a, PR_D, it0, (unsigned)T.col),
                               cprof<C>(a, PR_J33, it0, (unsigned)T.col), w6[3][3], frcp(w6[0][3]));
-    FaceLoop<C, 0>::template zf<6, 0>(w6, gz, W, T.omb);
+    FaceLoop<C, 0>::template zf<6, 0>(w6, gz[0], W, T.omb);
     pp[2] = pprime<C>(a, w6[4][2], T.mfac(a, w6[0][2], C::NM > 0 ? w6[C::IQV_SAFE][2] : 0.f), it0 - 1, (unsigned)T.col);
   };
   if (C::NM > 0 && !C::TERR && it0 > 0) {
@@ -1777,15 +1821,19 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
       const float Dz = C::TERR ? 1.f : prof(a, PR_D, z2);
       const float hxD = 0.5f * a.dXi * Dz, hyD = 0.5f * a.dYi * Dz;
       {
-        float c[NF], fxn[NF], fy[NF];
+        if constexpr (C::REG) {
+          float c[NF], fxn[NF], fy[NF];
 #pragma unroll
-        for (int f = 0; f < NF; ++f) c[f] = win[f][4 + S];
-        own_faces<C>(rw, dr, ty, tx, c, C::TERR ? dr[ty + 1][tx + 1] : ri[S + 1], hxD, hyD, T.omb, fxn, fy);
+          for (int f = 0; f < NF; ++f) c[f] = win[f][4 + S];
+          own_faces<C>(rw, dr, ty, tx, c, C::TERR ? dr[ty + 1][tx + 1] : ri[S + 1], hxD, hyD, T.omb, fxn, fy);
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          gy[b2][f][ty][tx] = fy[f];
-          if constexpr (FXR) fx[S + 1][f] = fxn[f];
-          else gxo[b2][f][ty][tx] = fxn[f];
+          for (int f = 0; f < NF; ++f) {
+            gy[b2][f][ty][tx] = fy[f];
+            if constexpr (FXR) fx[S + 1][f] = fxn[f];
+            else gxo[b2][f][ty][tx] = fxn[f];
+          }
+        } else {
+          own_faces_lds<C>(rw, dr, ty, tx, hxD, hyD, T.omb, gx[b2], gy[b2]);
         }
       }
       /* ring faces, all fields per job row (splitting them over more waves costs more issue
@@ -1793,7 +1841,7 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
       {
         int i;
         if (on_job(PL.rfy[0], wave, lane, i)) ring_faces_y<C, 0, NF>(rw, gy[b2], dr, i, hyD, T.omb);
-        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, NF>(rw, gxr[b2], dr, i, hxD, T.omb);
+        if (on_job(PL.rfx[0], wave, lane, i)) ring_faces_x<C, 0, NF>(rw, gx[b2], dr, i, hxD, T.omb);
       }
     }
 
@@ -1807,20 +1855,27 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
 #pragma unroll
         for (int j = 0; j < 7; ++j) w7[f][j] = wv[f][j + S];
       float xr[NFP];
+      if constexpr (C::REG)
 #pragma unroll
-      for (int f = 0; f < NFP; ++f) xr[f] = f < NF ? ((const SRD *)gxr[b1][ty])[f] : 0.f;
+        for (int f = 0; f < NFP; ++f) xr[f] = f < NF ? ((const SRD *)gx[b1].g[ty])[f] : 0.f;
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         const SRD *py = (const SRD *)&gy[b1][f][ty][tx];
-        float px;
-        if constexpr (FXR) px = fx[S][f];
-        else px = ((const SRD *)&gxo[b1][f][ty][tx])[0];
-        dxy[f] = (lane_up(px, xr[f], tx) - px) + (py[TX] - py[0]);
+        if constexpr (C::REG) {
+          float px;
+          if constexpr (FXR) px = fx[S][f];
+          else px = ((const SRD *)&gxo[b1][f][ty][tx])[0];
+          dxy[f] = (lane_up(px, xr[f], tx) - px) + (py[TX] - py[0]);
+        } else {
+          const SRD *px = (const SRD *)&gx[b1].g[f][ty][tx];
+          dxy[f] = (px[1] - px[0]) + (py[TX] - py[0]);
+        }
       }
       dyn_tendency<C, 7>(a, z3, C::TERR ? trow : dyn_rows<C>(a, z3, (unsigned)T.col), w7, ri[S], ri[S + 1], pp[S], pp[S + 2], pg[S][0], pg[S][1],
-                         dxy, gz, gzhi, T.omb, F);
+                         dxy, gz[GZS ? S : 0], GZS ? gz[GZS ? S + 1 : 0] : gzhi, T.omb, F);
+      if constexpr (!GZS)
 #pragma unroll
-      for (int f = 0; f < NF; ++f) gz[f] = gzhi[f];
+        for (int f = 0; f < NF; ++f) gz[0][f] = gzhi[f];
       if (T.active) {
         float b0[NF];
 #pragma unroll
@@ -1828,6 +1883,9 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
         rk_store<C, EMIT>(a, T, o3, F, b0);
         if (a.pout) *(float *)((char *)a.pout + o3) = pp[S + 1];
       }
+    } else if constexpr (GZS) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) gz[S + 1][f] = gz[S][f];
     }
     __syncthreads();
   };
@@ -1844,6 +1902,7 @@ __device__ __forceinline__ void stage_plain_body(const StepArgs &a, TilePos tp) 
       hv[0][f] = hv[2][f];
       hv[1][f] = hv[3][f];
       if constexpr (BSA) bs[0][f] = bs[2][f];
+      if constexpr (GZS) gz[0][f] = gz[2][f];
       if constexpr (FXR) fx[0][f] = fx[2][f];
     }
     pp[0] = pp[2]; pp[1] = pp[3]; pp[2] = pp[4];
