@@ -588,7 +588,7 @@ int fe_sgs_enable(int on, float gate) {
       HIPCHK(hipMalloc(&G.tauL, 9 * ncell * sizeof(float)));
       HIPCHK(hipMalloc(&G.gmax, ncell * sizeof(float)));
       HIPCHK(hipMalloc(&G.mask, ncell));
-      HIPCHK(hipMalloc(&G.grad, 12 * ncell * sizeof(float)));
+      HIPCHK(hipMalloc(&G.grad, 10 * ncell * sizeof(float)));
       G.ncell_cap = ncell;
     }
     if (G.j33) HIPCHK(hipFree(G.j33));

@@ -478,12 +478,15 @@ __global__ void k_sgs_finish(const float *Y, const float *ymu, const float *ysd,
  * increasing order, FP32 bias and GELU) are those of the unfused kernels, so both paths give
  * the same bits.
  * What bounds it: vector instructions, 970 per wave and tile (600 of them the GELUs), at two waves
- * per SIMD (the prefetched features and the weights are 128 registers), then its gathers.
- * 128 x 128 x 48: 234 us with four lanes per cell that read each feature's normalisation from LDS,
- * stored it as two bytes and waited for every neighbour's loads, and a serial finish by one wave;
- * 170 us without, 164 us with the gradients by component (k_sgs_grad) instead of in records of 12
- * floats.  A contiguous run of tiles per XCD made no difference (170 us), nor did scalar
- * normalisation operands; chaining the layers in registers, a wave per 16 cells, was slower (180 us). */
+ * per SIMD (the prefetched features and the weights are 128 registers; 256 in all, 29 spilled), then
+ * its gathers.  128 x 128 x 48: 234 us with four lanes per cell that read each feature's normalisation
+ * from LDS, stored it as two bytes and waited for every neighbour's loads, and a serial finish by one
+ * wave; 170 us without, 158 us with the gradients by component (k_sgs_grad) instead of in records of
+ * 12 floats.  A contiguous run of tiles per XCD made no difference (170 us), nor did scalar
+ * normalisation operands; chaining the layers in registers, a wave per 16 cells, was slower (180 us).
+ * Three waves per SIMD, the features loaded in two halves (168 registers, 44 spilled): 161 us, and a
+ * 64 x 64 x 48 step 145 us against 132 (one tile per work-group, nothing to overlap); the halves at two
+ * waves (218, none spilled): 165 us, 131. */
 constexpr int FT = 64;
 
 struct FusedArgs {
@@ -533,13 +536,13 @@ struct TileCell {
 /* One wave's share of a tile's features, W the wave: features 64 W .. 64 W + 63, lane = cell.
  * Waves 0 to 2 need components of eight neighbours from their first on, wave 3 the last six
  * neighbours and the seven dtheta/dz. */
-template <int W, int H>
+template <int W>
 struct TileFeatures {
-  static constexpr int Q0 = 64 * W + 32 * H, N0 = Q0 / 9, NN = (Q0 + 31 < 243 ? Q0 + 31 : 242) / 9 - N0 + 1, TH = 9 * NN;
+  static constexpr int N0 = SGS_H * W / 9, NN = W < 3 ? 8 : 6, TH = 9 * NN;
   static_assert(SGS_H == FT && SGS_KIN == 4 * FT, "64 features per wave");
-  static_assert(TH + (Q0 + 31 < 243 ? 0 : 7) <= 45, "a half's features fit");
-  __device__ __forceinline__ static void load(const FusedArgs &a, const TileCell &p, float (&u)[45], float &rho) {
-    if (H == 0) rho = a.S[(long)p.z * a.ps + (long)p.y * a.P + p.x];
+  static_assert(W == 3 || 9 * (N0 + NN) >= 64 * (W + 1), "the neighbours hold the wave's features");
+  __device__ __forceinline__ static void load(const FusedArgs &a, const TileCell &p, float (&u)[72], float &rho) {
+    if (W == 0) rho = a.S[(long)p.z * a.ps + (long)p.y * a.P + p.x];
     /* a neighbour's place is the cell's plus one step per direction, wrapped or clamped by the step
      * (32 bits, modulo 2^32: the sum is a place in the grid) */
     const unsigned c = (unsigned)p.c, row = (unsigned)a.Nx, plane = row * (unsigned)a.Ny;
@@ -558,7 +561,7 @@ struct TileFeatures {
       u[9 * i + 4] = u1.x; u[9 * i + 5] = u1.y; u[9 * i + 6] = u1.z; u[9 * i + 7] = u1.w;
       u[9 * i + 8] = gc[id];
     }
-    if constexpr (W == 3 && H == 1) {
+    if constexpr (W == 3) {
       /* dtheta/dz of the cell, x-, x+, y-, y+, z-, z+ (c_sgs_tnb) */
       const float *gt = gc + a.ncell;
       u[TH + 0] = gt[cell(0, 0, 0)];
@@ -570,45 +573,42 @@ struct TileFeatures {
       u[TH + 6] = gt[cell(0, 0, 1)];
       /* the same last element in every wave's branch: the array stays in registers */
 #pragma unroll
-      for (int i = TH + 7; i < 45; ++i) u[i] = 0.f;
-    } else {
-#pragma unroll
-      for (int i = TH; i < 45; ++i) u[i] = 0.f;
+      for (int i = TH + 7; i < 72; ++i) u[i] = 0.f;
     }
   }
   /* normalised, to As; returns their largest magnitude */
-  __device__ __forceinline__ static float put(const float2 *nrm, const float (&u)[45], uint2 (*As)[FT], int lane) {
+  __device__ __forceinline__ static float put(const float2 *nrm, const float (&u)[72], uint2 (*As)[FT], int lane) {
     float gm = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (Q0 + 4 * i >= SGS_NIN) break;
+    for (int i = 0; i < 16; ++i) {
       if (i > 0 && i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
       float v[4];
-      const float4 n01 = *(const float4 *)&nrm[Q0 + 4 * i], n23 = *(const float4 *)&nrm[Q0 + 4 * i + 2];
+      const float4 n01 = *(const float4 *)&nrm[64 * W + 4 * i], n23 = *(const float4 *)&nrm[64 * W + 4 * i + 2];
       const float mu[4] = {n01.x, n01.z, n23.x, n23.z}, isd[4] = {n01.y, n01.w, n23.y, n23.w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int q = Q0 + 4 * i + j;
+        const int q = 64 * W + 4 * i + j;
         if (q < SGS_NIN) {
           const int k = q < 243 ? q - 9 * N0 : TH + q - 243;
-          v[j] = (u[k < 45 ? k : 0] - mu[j]) * isd[j];
+          v[j] = (u[k < 72 ? k : 0] - mu[j]) * isd[j];
           gm = fmaxf(gm, fabsf(v[j]));
         } else {
           v[j] = 0.f;
         }
       }
-      As[Q0 / 4 + i][lane] = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+      As[16 * W + i][lane] = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
     }
     return gm;
   }
 };
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) k_sgs_mlp_fused(FusedArgs a) {
-  __shared__ uint2 As[(SGS_NIN + 3) / 4][FT];  /* features     [k / 4][cell][4]; k >= 252 are 0 */
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_sgs_mlp_fused(FusedArgs a) {
+  __shared__ uint2 As[SGS_KIN / 4][FT];        /* features     [k / 4][cell][4] */
   __shared__ uint2 Hs[2][SGS_H / 4][FT];       /* activations, likewise */
-  __shared__ float gms[2][4][FT];              /* by tile parity: each wave's largest feature */
+  __shared__ float gms[2][4][FT], rhos[2][FT]; /* by tile parity: each wave's largest feature, rho */
   __shared__ __align__(16) float cf[4][SGS_H]; /* biases of layers 1-3; of layer 4, output std, output mean */
-  __shared__ __align__(16) float2 nrm[(SGS_NIN + 3) / 4 * 4];  /* feature normalisation: mean, 1 / std */
+  __shared__ __align__(16) float2 nrm[SGS_KIN];  /* feature normalisation: mean, 1 / std */
+  __shared__ unsigned cnts[4][2];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
   /* weights as the left operand (its row = output column): lane holds W[k = 16 kb + 4 lk + v][n],
@@ -631,39 +631,35 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
     w4[kb] = bf16x4{(short)f2bf(a.w[OW4_ + (k + 0) * SGS_KOUT + lr]), (short)f2bf(a.w[OW4_ + (k + 1) * SGS_KOUT + lr]),
                     (short)f2bf(a.w[OW4_ + (k + 2) * SGS_KOUT + lr]), (short)f2bf(a.w[OW4_ + (k + 3) * SGS_KOUT + lr])};
   }
-  for (int i = tid; i < (SGS_NIN + 3) / 4 * 4; i += 256) nrm[i] = make_float2(a.mu[i], a.isd[i]);
+  for (int i = tid; i < SGS_KIN; i += 256) nrm[i] = make_float2(a.mu[i], a.isd[i]);
   for (int i = tid; i < SGS_H; i += 256) {
     cf[0][i] = a.w[OB1_ + i];
     cf[1][i] = a.w[OB2_ + i];
     cf[2][i] = a.w[OB3_ + i];
     cf[3][i] = i < SGS_KOUT ? a.w[OB4_ + i] : i < 2 * SGS_KOUT ? a.ysd[i - SGS_KOUT] : i < 3 * SGS_KOUT ? a.ymu[i - 2 * SGS_KOUT] : 0.f;
   }
-  float u[45], rho = 0.f, gm = 0.f;                /* the wave's raw features of a tile (TileFeatures), rho (wave 0) */
+  float u[72], rho = 0.f;                /* the wave's raw features of a tile (TileFeatures), rho (wave 0) */
 #pragma unroll
-  for (int i = 0; i < 45; ++i) u[i] = 0.f;
+  for (int i = 0; i < 72; ++i) u[i] = 0.f;
   TileCell p(a, (long)blockIdx.x * FT + lane);
   const long step = (long)gridDim.x * FT;
   int sx, sy, sz;
   cell_xyz(step, a.Nx, a.Ny, sx, sy, sz);
-  auto load = [&](auto half) {
-    constexpr int H = decltype(half)::value;
-    if (wave == 0) TileFeatures<0, H>::load(a, p, u, rho);
-    else if (wave == 1) TileFeatures<1, H>::load(a, p, u, rho);
-    else if (wave == 2) TileFeatures<2, H>::load(a, p, u, rho);
-    else TileFeatures<3, H>::load(a, p, u, rho);
+  auto load = [&]() {
+    if (wave == 0) TileFeatures<0>::load(a, p, u, rho);
+    else if (wave == 1) TileFeatures<1>::load(a, p, u, rho);
+    else if (wave == 2) TileFeatures<2>::load(a, p, u, rho);
+    else TileFeatures<3>::load(a, p, u, rho);
   };
-  auto put = [&](auto half, int buf) {
-    constexpr int H = decltype(half)::value;
-    float g;
-    if (wave == 0) g = TileFeatures<0, H>::put(nrm, u, As, lane);
-    else if (wave == 1) g = TileFeatures<1, H>::put(nrm, u, As, lane);
-    else if (wave == 2) g = TileFeatures<2, H>::put(nrm, u, As, lane);
-    else g = TileFeatures<3, H>::put(nrm, u, As, lane);
-    if (H == 0) gm = g;
-    else gms[buf][wave][lane] = fmaxf(gm, g);
+  auto put = [&](int buf) {
+    float gm;
+    if (wave == 0) gm = TileFeatures<0>::put(nrm, u, As, lane);
+    else if (wave == 1) gm = TileFeatures<1>::put(nrm, u, As, lane);
+    else if (wave == 2) gm = TileFeatures<2>::put(nrm, u, As, lane);
+    else gm = TileFeatures<3>::put(nrm, u, As, lane);
+    gms[buf][wave][lane] = gm;
+    if (wave == 0) rhos[buf][lane] = rho;
   };
-  const std::integral_constant<int, 0> h0;
-  const std::integral_constant<int, 1> h1;
   f32x4 acc[4];
   auto product = [&](const uint2 (*src)[FT], const bf16x4 *w, int nkb) {
 #pragma unroll
@@ -673,7 +669,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
       if (kb > 0 && kb % 4 == 0) __builtin_amdgcn_sched_barrier(0);   /* 16 operand reads in flight, no more registers */
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
-        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w[kb], kb == 15 && lk == 3 ? bf16x4{0, 0, 0, 0} : ld_frag(&src[4 * kb + lk][16 * rb + lr]), acc[rb], 0, 0, 0);
+        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w[kb], ld_frag(&src[4 * kb + lk][16 * rb + lr]), acc[rb], 0, 0, 0);
     }
   };
   auto store_act = [&](int buf, int layer) {
@@ -687,33 +683,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
   unsigned ncnt = 0, npass = 0;          /* cells finished and passing, by lanes 0..15 of each wave */
   int buf = 0;
   if ((int)blockIdx.x < a.ntiles) {
-    load(h0);
+    load();
     __syncthreads();                     /* nrm, cf */
-    put(h0, 0);
-    load(h1);
-    put(h1, 0);
+    put(0);
   }
   for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x, buf ^= 1) {
     const int next = tile + gridDim.x;
     __syncthreads();
-    const float rhoc = rho;                /* of this tile */
     if (next < a.ntiles) {
       p.advance(a, step, sx, sy, sz);
-      load(h0);
+      load();
     }
     product(As, w1, 16);
     store_act(0, 0);
     __syncthreads();
-    if (next < a.ntiles) {
-      put(h0, buf ^ 1);
-      load(h1);
-    }
+    if (next < a.ntiles) put(buf ^ 1);
     product(Hs[0], w2, 4);
     store_act(1, 1);
     __syncthreads();
     product(Hs[1], w3, 4);
     store_act(0, 2);
-    if (next < a.ntiles) put(h1, buf ^ 1);
     __syncthreads();
     /* ---- layer 4 and finish: wave w the cell block w, the lane's outputs 4 lk .. 4 lk + 3 ---- */
     f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -722,7 +711,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
       o = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w4[kb], ld_frag(&Hs[0][4 * kb + lk][16 * wave + lr]), o, 0, 0, 0);
     const int r = 16 * wave + lr;
     const long c = (long)tile * FT + r;
-    const float rc = __shfl(rhoc, r);
+    const float rc = rhos[buf][r];
     float t[4];
     const float *b4 = &cf[3][4 * lk], *ysd = b4 + SGS_KOUT, *ymu = ysd + SGS_KOUT;
 #pragma unroll
@@ -750,16 +739,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
     ncnt += __shfl_xor(ncnt, off);
     npass += __shfl_xor(npass, off);
   }
-  unsigned *cnt = (unsigned *)&gms[0][0][0];
-  __syncthreads();
   if (lane == 0) {
-    cnt[2 * wave] = ncnt;
-    cnt[2 * wave + 1] = npass;
+    cnts[wave][0] = ncnt;
+    cnts[wave][1] = npass;
   }
   __syncthreads();
   if (tid == 0 && (int)blockIdx.x < a.ntiles) {
-    atomicAdd(&a.count[0], (unsigned long long)(cnt[0] + cnt[2] + cnt[4] + cnt[6]));
-    atomicAdd(&a.count[1], (unsigned long long)(cnt[1] + cnt[3] + cnt[5] + cnt[7]));
+    atomicAdd(&a.count[0], (unsigned long long)(cnts[0][0] + cnts[1][0] + cnts[2][0] + cnts[3][0]));
+    atomicAdd(&a.count[1], (unsigned long long)(cnts[0][1] + cnts[1][1] + cnts[2][1] + cnts[3][1]));
   }
 }
 
