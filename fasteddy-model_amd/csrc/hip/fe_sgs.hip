@@ -506,7 +506,18 @@ int fe_sgs_norm(float *buf, long n, int get) {
   return FE_OK;
 }
 
-/* n floats of a caller's rows to the device */
+/* The network stream, waited for on every way out of a call that has handed it host memory. */
+struct SgsDone {
+  bool waited = false;
+  int wait() {
+    waited = true;
+    HIPCHK(hipStreamSynchronize(sgs_stream()));
+    return FE_OK;
+  }
+  ~SgsDone() { if (!waited) (void)hipStreamSynchronize(sgs_stream()); }
+};
+
+/* n floats of a caller's rows to the device; read when the stream is done (SgsDone) */
 static int sgs_rows_up(float *dev, const float *host, long n) {
   const size_t bytes = n * sizeof(float);
   int rc;
@@ -526,11 +537,11 @@ int fe_mlp_forward(const float *X, long M, float *Y) {
   if (!X || !Y || M < 1) return FE_ERR_UNSUPPORTED;
   if (!G.have_w) return FE_ERR_STATE;
   if ((rc = sgs_rows(M))) return rc;
+  SgsDone done;
   if ((rc = sgs_rows_up(G.Xb, X, M * SGS_KIN))) return rc;
   if ((rc = mlp_forward(G.Xb, M))) return rc;
   HIPCHK(hipMemcpyAsync(Y, G.Y, M * SGS_KOUT * sizeof(float), hipMemcpyDeviceToHost, sgs_stream()));
-  HIPCHK(hipStreamSynchronize(sgs_stream()));
-  return FE_OK;
+  return done.wait();
 }
 
 /* Gradient of the training loss (mean squared error over the first 9 of the 16 output
@@ -542,16 +553,17 @@ int fe_mlp_gradient(const float *X, const float *T, long M, float *grad, double 
   if (!G.have_w) return FE_ERR_STATE;
   if ((rc = sgs_rows(M))) return rc;
   hipStream_t s = sgs_stream();
+  double l = 0.0;
+  SgsDone done;
   if ((rc = sgs_rows_up(G.Xb, X, M * SGS_KIN))) return rc;
   if ((rc = sgs_rows_up(G.Tb, T, M * SGS_KOUT))) return rc;
   HIPCHK(hipMemsetAsync(G.dloss, 0, sizeof(double), s));
   if ((rc = mlp_forward(G.Xb, M))) return rc;
   if ((rc = sgs_loss_grad(G.Tb, M))) return rc;
   if ((rc = mlp_backward(G.Xb, M))) return rc;
-  double l = 0.0;
   HIPCHK(hipMemcpyAsync(grad, G.gw, NPARAM * sizeof(float), hipMemcpyDeviceToHost, s));
   if (loss) HIPCHK(hipMemcpyAsync(&l, G.dloss, sizeof(double), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
+  if ((rc = done.wait())) return rc;
   if (loss) loss[0] = l / ((double)M * SGS_NOUT);
   return FE_OK;
 }
