@@ -124,7 +124,8 @@ int fe_ens_member_info(int m, int *info, int n);
 int fe_ens_member_state(int m, float *out, long n);
 /* Member friction velocity ([y][x], pitch P), n = Ny*P floats. */
 int fe_ens_member_ustar(int m, float *out, long n);
-/* z segments of member m (work tile 64 x 8 x ceil(Nz/nseg) levels). */
+/* z segments of member m (work tile 64 x 8 x ceil(Nz/nseg) levels).  Members that are given none, by this
+ * or by amd_zSegments, share a segment length chosen for all members together, again whenever one is added. */
 int fe_ens_set_segments(int m, int nseg);
 /* nsteps RK3 steps of every member (graph replays, one synchronisation). */
 int fe_ens_steps(int nsteps);
